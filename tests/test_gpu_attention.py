@@ -466,6 +466,59 @@ def test_long_prompt_prefill_block_sizes(kernel, dev, bs, window, dtype, d):
         torch.testing.assert_close(got[cu[s]:cu[s + 1]].float(), want, atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("dtype,kv,d,hq,hkv", [(torch.bfloat16, "same", 128, 4, 2),
+                                               (torch.float16, "same", 96, 2, 2),
+                                               (torch.bfloat16, "same", 64, 3, 1),
+                                               (torch.bfloat16, "fp8", 128, 2, 1),
+                                               (torch.float16, "fp8_vector", 64, 2, 2)])
+def test_prefill_tiling_at_tile_edges(kernel, dev, dtype, kv, d, hq, hkv):
+    """The prefill tiling's tile loop runs two 64-position tiles a turn with K one tile
+    ahead of V: windows ending on, before and past each of the first tiles (one, two,
+    three and four tiles, an odd and an even number of turns), row groups of one row and
+    of 128, windows longer than their context (rows that see nothing give zeros), NaN in
+    every pool position no row may see, against dense fp32 attention.  Tolerance as the
+    other 16-bit attention tests (weights and output rounded to 16 bits)."""
+    _say("prefill tile edges", dtype, kv, d)
+    g = torch.Generator().manual_seed(31 + d)
+    bs = 16
+    seqs = [(64, 64), (65, 65), (127, 64), (128, 128), (129, 100), (191, 70), (192, 1), (193, 65),
+            (256, 129), (257, 66), (20, 33), (0, 3)]  # (context, window)
+    pages = sum(-(-n // bs) for n, _ in seqs) + 1
+    fp8 = kv != "same"
+    pool_dtype = torch.float8_e4m3fn if fp8 else dtype
+    k_f, v_f = (torch.randn(pages, bs, hkv, d, generator=g) for _ in range(2))
+    scale = {"same": torch.tensor(1.0), "fp8": torch.tensor(0.02),
+             "fp8_vector": torch.rand(pages, bs, hkv, generator=g) * 0.02 + 0.01}[kv]
+    s4 = scale.unsqueeze(-1) if scale.ndim else scale
+    k, v = (k_f / s4).to(pool_dtype), (v_f / s4).to(pool_dtype)
+    k_deq, v_deq = k.float() * s4, v.float() * s4
+    tables = random_tables([n for n, _ in seqs], bs, pages, g)
+    seen = torch.zeros(pages, bs, dtype=torch.bool)
+    for s, (n, _) in enumerate(seqs):
+        for pos in range(n):
+            seen[tables[s, pos // bs], pos % bs] = True
+    for pool in (k, v):
+        bits = pool.view(torch.uint8 if fp8 else torch.int16)
+        bits[~seen] = 0x7F if fp8 else 0x7FFF  # a NaN of each type
+    total = sum(c for _, c in seqs)
+    q = torch.randn(total, hq, d, generator=g).to(dtype)
+    lengths = torch.tensor([n for n, _ in seqs], dtype=torch.int32)
+    cu = torch.tensor([0] + list(torch.tensor([c for _, c in seqs]).cumsum(0)), dtype=torch.int32)
+    scales = (None, None) if kv == "same" else (scale.to(dev), scale.to(dev))
+    got = kernel.prefill(q.to(dev), k.to(dev), v.to(dev), tables.to(dev), lengths.to(dev),
+                         cu.to(dev), max(c for _, c in seqs), *scales).cpu()
+    for s, (n, c) in enumerate(seqs):
+        rows = got[cu[s]:cu[s + 1]].float()
+        blind = max(0, c - n)  # rows before the first position see nothing
+        assert torch.equal(rows[:blind], torch.zeros_like(rows[:blind]))
+        if c > blind:
+            pages_s = tables[s, : -(-n // bs)].long()
+            want = _dense_packed(q[cu[s] + blind:cu[s + 1]],
+                                 k_deq[pages_s].reshape(-1, hkv, d)[:n],
+                                 v_deq[pages_s].reshape(-1, hkv, d)[:n], c - blind, n)
+            torch.testing.assert_close(rows[blind:], want, atol=2e-2, rtol=2e-2)
+
+
 # ------------------------------------------ packed rows with explicit row lengths
 
 def _group_rows_by_plane(n, w, planes, d0, row_len, order="ascending"):

@@ -281,21 +281,17 @@ struct Flag {
   static constexpr bool value = B;
 };
 
-// Four fp8 codes -> four 16-bit values of the MFMA type (exact for e4m3).
+// Four fp8 codes -> four 16-bit values of the MFMA type (exact for e4m3; two gfx950
+// pair conversions, where the way through fp32 took four and the packing).
 template <int QT>
 __device__ __forceinline__ uint2 fp8x4_to_16(uint32_t w) {
-  const float2 lo = fp8x2_to_f32<false>(w);
-  const float2 hi = fp8x2_to_f32<true>(w);
-  uint2 r;
-  if (QT == RLT_BF16) {
-    // e4m3 values are exact in bf16: truncation of the fp32 bits is exact.
-    r.x = (__float_as_uint(lo.x) >> 16) | (__float_as_uint(lo.y) & 0xffff0000u);
-    r.y = (__float_as_uint(hi.x) >> 16) | (__float_as_uint(hi.y) & 0xffff0000u);
-  } else {
-    r.x = (uint32_t)f32_to_f16_bits(lo.x) | ((uint32_t)f32_to_f16_bits(lo.y) << 16);
-    r.y = (uint32_t)f32_to_f16_bits(hi.x) | ((uint32_t)f32_to_f16_bits(hi.y) << 16);
-  }
-  return r;
+  if (QT == RLT_BF16)
+    return make_uint2(
+        __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.f, false)),
+        __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.f, true)));
+  return make_uint2(
+      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.f, false)),
+      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.f, true)));
 }
 
 // One lane's raw key elements, as loaded from HBM: for contraction step s the
@@ -1444,431 +1440,7 @@ __global__ __launch_bounds__(256) void rlt_merge_kernel(AttnParams P) {
   }
 }
 
-// ============================================================ long-prompt prefill
-//
-// Calls whose longest q window reaches kPfMinQ rows (prompt prefill, long chunks)
-// take a tiling built for many rows per sequence: one 256-thread workgroup per
-// (sequence, 128-row group, kv head), each wave owning 32 rows (two 16-row MFMA
-// tiles).  64-position K and V tiles are staged once per workgroup in LDS (K as
-// [position][dim], V transposed to [dim][position] while it is stored) and shared
-// by the four waves, double-buffered with the next tile's global loads in
-// registers.  The math is the verify kernel's (S^T = K Q^T, online softmax in the
-// log2 domain, O^T = V^T P^T), with both products on v_mfma_f32_16x16x32: the
-// P^T operand of a key-tile pair is the two S^T accumulators of the lane, and the
-// contraction order over the pair's 32 positions is permuted to match.  The
-// output is normalized in the kernel (no split, no merge launch).  Rows of such a
-// call are equal to the per-row form within floating-point tolerance, not bit for
-// bit (the tile boundaries differ).
-constexpr int kPfNT = 2;        // 16-row MFMA tiles per wave
-constexpr int kPfWaves = 4;     // waves per workgroup (sharing each staged tile)
-constexpr int kPfRows = kPfWaves * 16 * kPfNT;  // q rows per workgroup
-constexpr int kPfKeys = 64;     // key positions per LDS tile
-constexpr int kPfThreads = 64 * kPfWaves;
-constexpr int kPfMinQ = 64;     // q window length from which a call takes this path
-constexpr float kPfLazy = 8.f;  // log2 headroom before the running max moves
-
-// LDS row width in dims: D = 96 rows take a 128-dim row whose last four 16-byte slots
-// (their place moves with the swizzle) are never loaded nor read
-template <int D>
-constexpr int pf_row_dims() { return D == 96 ? 128 : D; }
-
-template <int D>
-struct PrefillLds {
-  static constexpr int kRowB = pf_row_dims<D>() * 2;  // bytes per position row (XOR-swizzled slots)
-  uint8_t k[2][kPfKeys * kRowB];
-  uint8_t v[2][kPfKeys * kRowB];
-  float ks[2][kPfKeys];  // per-vector fp8 scales of the tile's positions (SM 2)
-  float vs[2][kPfKeys];
-};
-
-typedef __attribute__((address_space(3))) void lds_void;
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-
-// 16-byte slot of piece `piece` (8 dims) in row r of a staged tile.  K rows XOR the
-// slot with r mod SLOTS, so the S^T operand reads (16 lanes = 16 rows of one piece
-// column) meet distinct bank groups; V rows XOR it with 2 (r & 3), which keeps each piece
-// pair adjacent for the transpose reads (16 lanes = 4 rows x one 32-byte pair) and puts
-// the four rows on distinct bank groups, and with 8 in rows with bit 2 set (16 slots), so
-// the next 16 lanes (rows 4 further on) use the other half of the banks.
-template <int SLOTS>
-__device__ __forceinline__ int k_slot(int r, int piece) { return piece ^ (r & (SLOTS - 1)); }
-template <int SLOTS>
-__device__ __forceinline__ int v_slot(int r, int piece) {
-  return piece ^ (2 * (r & 3)) ^ (SLOTS >= 16 ? 8 * ((r >> 2) & 1) : 0);
-}
-
-// UB: block_size % 16 == 0, so each 16-position group of a tile lies in one block
-// and its address comes from one wave-uniform table lookup (16-bit pools).
-// KVT: the pool type, QT's own or fp8-e4m3 with scale mode SM (1 per-tensor, 2
-// per-vector).  FP8 tiles are staged through registers: each thread loads 8-code pieces
-// (item e = 256 j + t: LDS slot e % SLOTS of row e / SLOTS, holding the piece the
-// swizzle puts there) while the previous tile is in use, then widens them to QT (exact
-// for e4m3) into the same swizzled LDS layout, each wave writing contiguous slots; the
-// per-tensor key scale folds into the score scale and the value scale into the output,
-// per-vector scales multiply each position's score and (for P V only) its weight.
-template <int QT, int KVT, int D, int SM, bool UB>
-__global__ __launch_bounds__(kPfThreads, kPfNT > 2 || kPfWaves > 4 ? 1 : 2) void rlt_prefill_kernel(AttnParams P) {
-  using M = Mfma<QT>;
-  using L = PrefillLds<D>;
-  constexpr int NT = kPfNT;
-  constexpr int NQS = D / 32;       // 32-wide contraction slices of S^T
-  constexpr int ND = D / 16;        // 16-wide dim tiles of O^T
-  constexpr int PIECES = D / 8;     // 16-byte pieces of a position row in the pool
-  constexpr int SLOTS = pf_row_dims<D>() / 8;  // 16-byte slots per LDS row (>= PIECES)
-  constexpr int ROWS_PER_LD = 64 / SLOTS;                // rows one wave-wide direct load fills
-  constexpr int LDS_PER_WAVE = kPfKeys / ROWS_PER_LD / kPfWaves;  // direct loads per wave per tile (K, V each)
-  static_assert(LDS_PER_WAVE * ROWS_PER_LD * kPfWaves == kPfKeys, "the waves' loads cover a tile");
-  static_assert(16 % ROWS_PER_LD == 0, "a direct load's rows stay in one 16-position group");
-  constexpr bool FP8 = KVT != QT;
-  static_assert(!FP8 || KVT == RLT_FP8_E4M3, "16-bit pools match q");
-  static_assert(FP8 == (SM != 0), "scale modes are for fp8 pools");
-  constexpr int FJ = kPfKeys * SLOTS / kPfThreads;  // fp8 LDS slots per thread per tile (K, V each)
-  static_assert(FJ * kPfThreads == kPfKeys * SLOTS, "the threads' fp8 slots cover a tile");
-  __shared__ L sh;
-  const int t = threadIdx.x, w = t >> 6, lane = t & 63, l16 = lane & 15, grp = lane >> 4;
-
-  // heaviest row-groups (latest positions) first across the whole batch: the
-  // row-group index is outermost, then the sequence, then the kv head
-  const int64_t id = blockIdx.x;
-  const int kvh = (int)(id % P.hkv);
-  const int64_t sr = id / P.hkv;
-  const int seq = (int)(sr % P.num_seqs);
-  const int rg = P.rowgroups - 1 - (int)(sr / P.num_seqs);
-  const SeqView sv = seq_view(P, seq);
-  const int rows_total = sv.q_len * P.group;
-  const int rg_begin = rg * kPfRows;
-  if (rg_begin >= rows_total) return;  // uniform over the workgroup
-  const int rg_rows = min(kPfRows, rows_total - rg_begin);
-  int lo_first, hi_first, lo_last, hi_last;
-  group_range(P, sv, rg_begin, rg_rows, lo_first, hi_first, lo_last, hi_last);
-
-  // this lane's rows (one per 16-row tile): B operand of S^T = K Q^T
-  uint4 qreg[NT][NQS];
-  int row_lo[NT], row_hi[NT];
-  // the wave's common visible range: tiles inside [wlo, whi) need no position masks
-  // (rows past the group are not stored and do not narrow it)
-  int wlo = -(1 << 30), whi = 1 << 30;
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int local = w * 16 * NT + nt * 16 + l16;
-    if (local < rg_rows) {
-      const int rho = rg_begin + local;
-      const int qi = rho / P.group;
-      const int head = kvh * P.group + rho % P.group;
-      row_range(P, sv, qi, row_lo[nt], row_hi[nt]);
-      wlo = max(wlo, row_lo[nt]);
-      whi = min(whi, row_hi[nt]);
-      const uint16_t* qp = (const uint16_t*)P.q + (int64_t)(sv.q_begin + qi) * P.q_row_stride +
-                           (int64_t)head * P.q_head_stride + grp * 8;
-#pragma unroll
-      for (int s = 0; s < NQS; ++s) qreg[nt][s] = *(const uint4*)(qp + 32 * s);
-    } else {
-      row_lo[nt] = row_hi[nt] = 0;
-#pragma unroll
-      for (int s = 0; s < NQS; ++s) qreg[nt][s] = make_uint4(0, 0, 0, 0);
-    }
-  }
-  for (int off = 32; off >= 1; off >>= 1) {
-    wlo = max(wlo, __shfl_xor(wlo, off, RLT_WAVE));
-    whi = min(whi, __shfl_xor(whi, off, RLT_WAVE));
-  }
-  wlo = __builtin_amdgcn_readfirstlane(wlo);
-  whi = __builtin_amdgcn_readfirstlane(whi);
-
-  f32x4 oacc[NT][ND];
-  float m_run[NT], l_run[NT];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    m_run[nt] = -INFINITY;
-    l_run[nt] = 0.f;
-#pragma unroll
-    for (int dt = 0; dt < ND; ++dt) oacc[nt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-
-  // ---- global -> LDS staging of one 64-position tile by direct loads: wave w's j-th
-  // load fills rows ROWS_PER_LD (LDS_PER_WAVE w + j) + [0, ROWS_PER_LD); lane L takes row
-  // + L / SLOTS and LDS slot L % SLOTS, into which it loads the row's swizzled piece
-  const int ld_row = lane / SLOTS;
-  const int ld_slot = lane % SLOTS;
-  const int64_t k_head = (int64_t)kvh * P.k_head_stride;
-  const int64_t v_head = (int64_t)kvh * P.v_head_stride;
-  // (block id, offset) of position pos: block ids outside the pool read block 0
-  auto block_of = [&](int pos, int64_t& blk, int& off) {
-    const int idx = min(pos / P.block_size, P.table_width - 1);
-    const int32_t e = P.tables[(int64_t)seq * P.table_stride + idx];
-    blk = (e >= 0 && e < P.num_blocks) ? e : 0;
-    off = pos % P.block_size;
-  };
-  uint2 kraw[FP8 ? FJ : 1], vraw[FP8 ? FJ : 1];
-  float sraw = 0.f;
-  auto load = [&](int tile, int b) {
-    const int base = tile * kPfKeys;
-    if constexpr (FP8) {
-#pragma unroll
-      for (int j = 0; j < FJ; ++j) {
-        // item e: LDS slot e % SLOTS of row e / SLOTS, so each wave's LDS writes are
-        // contiguous (scattered 16-byte writes of permuted slots conflicted); the slot
-        // holds the row's piece k_slot / v_slot (an involution), loaded here
-        const int e = j * kPfThreads + t;
-        const int r = e / SLOTS, sl = e % SLOTS;
-        const int kpc = k_slot<SLOTS>(r, sl), vpc = v_slot<SLOTS>(r, sl);
-        int64_t blk;
-        int off;
-        block_of(base + r, blk, off);
-        if (PIECES == SLOTS || kpc < PIECES)
-          kraw[j] = *(const uint2*)((const uint8_t*)P.k + blk * P.k_block_stride +
-                                    (int64_t)off * P.k_token_stride + k_head + kpc * 8);
-        if (PIECES == SLOTS || vpc < PIECES)
-          vraw[j] = *(const uint2*)((const uint8_t*)P.v + blk * P.v_block_stride +
-                                    (int64_t)off * P.v_token_stride + v_head + vpc * 8);
-      }
-      if (SM == 2 && t < 2 * kPfKeys) {  // threads 0-63 key scales, 64-127 value scales
-        const int pos = base + (t & (kPfKeys - 1));
-        int64_t blk;
-        int off;
-        block_of(pos, blk, off);
-        const float x = (t < kPfKeys ? P.k_scale : P.v_scale)[blk * P.s_block_stride +
-                                                              (int64_t)off * P.s_token_stride +
-                                                              (int64_t)kvh * P.s_head_stride];
-        sraw = pos < hi_last ? x : 0.f;
-      }
-      return;
-    }
-#pragma unroll
-    for (int j = 0; j < LDS_PER_WAVE; ++j) {
-      const int r0 = ROWS_PER_LD * (LDS_PER_WAVE * w + j);  // wave-uniform
-      const int r = r0 + ld_row;
-      int64_t blk;
-      int off;
-      if (UB) {
-        block_of(__builtin_amdgcn_readfirstlane(base + (r0 & ~15)), blk, off);
-        off += r & 15;
-      } else {
-        block_of(base + r, blk, off);
-      }
-      // (the slot of lane ld_slot holds piece k_slot / v_slot of row r: an involution)
-      const int kpc = k_slot<SLOTS>(r, ld_slot);
-      const int vpc = v_slot<SLOTS>(r, ld_slot);
-      const uint16_t* kp = (const uint16_t*)P.k + blk * P.k_block_stride +
-                           (int64_t)off * P.k_token_stride + k_head + kpc * 8;
-      const uint16_t* vp = (const uint16_t*)P.v + blk * P.v_block_stride +
-                           (int64_t)off * P.v_token_stride + v_head + vpc * 8;
-      // padded rows: lanes whose slot holds a piece past the row load nothing
-      if (PIECES == SLOTS || kpc < PIECES)
-        __builtin_amdgcn_global_load_lds((const void*)kp, (lds_void*)(sh.k[b] + r0 * L::kRowB), 16, 0, 0);
-      if (PIECES == SLOTS || vpc < PIECES)
-        __builtin_amdgcn_global_load_lds((const void*)vp, (lds_void*)(sh.v[b] + r0 * L::kRowB), 16, 0, 0);
-    }
-  };
-  // After this wave's loads of tile `tile` into buffer b landed: its V rows past the
-  // sequence may hold any bits (NaN included) and are zeroed, since their weight 0
-  // times NaN would not vanish.  Only the tiles that reach past hi_last do work.
-  auto settle = [&](int tile, int b) {
-    const int base = tile * kPfKeys;
-    if constexpr (FP8) {
-#pragma unroll
-      for (int j = 0; j < FJ; ++j) {
-        const int e = j * kPfThreads + t;
-        const int r = e / SLOTS, sl = e % SLOTS;
-        // (pad slots of 96-dim rows are never read: left unwritten)
-        if (PIECES == SLOTS || k_slot<SLOTS>(r, sl) < PIECES) {
-          const uint2 k0 = fp8x4_to_16<QT>(kraw[j].x), k1 = fp8x4_to_16<QT>(kraw[j].y);
-          // two 8-byte halves: 16-byte LDS writes of a whole wave conflicted (the counters
-          // read 4x the cycles of an ideal write)
-          uint2* kd = (uint2*)(sh.k[b] + r * L::kRowB + sl * 16);
-          kd[0] = make_uint2(k0.x, k0.y);
-          kd[1] = make_uint2(k1.x, k1.y);
-        }
-        if (PIECES == SLOTS || v_slot<SLOTS>(r, sl) < PIECES) {
-          uint4 vx = make_uint4(0, 0, 0, 0);
-          if (base + r < hi_last) {
-            const uint2 v0 = fp8x4_to_16<QT>(vraw[j].x), v1 = fp8x4_to_16<QT>(vraw[j].y);
-            vx = make_uint4(v0.x, v0.y, v1.x, v1.y);
-          }
-          uint2* vd = (uint2*)(sh.v[b] + r * L::kRowB + sl * 16);
-          vd[0] = make_uint2(vx.x, vx.y);
-          vd[1] = make_uint2(vx.z, vx.w);
-        }
-      }
-      if (SM == 2 && t < 2 * kPfKeys) (t < kPfKeys ? sh.ks[b] : sh.vs[b])[t & (kPfKeys - 1)] = sraw;
-      return;
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (base + kPfKeys > hi_last) {
-#pragma unroll
-      for (int j = 0; j < LDS_PER_WAVE; ++j) {
-        const int r = ROWS_PER_LD * (LDS_PER_WAVE * w + j) + ld_row;
-        if (base + r >= hi_last)
-          *(uint4*)(sh.v[b] + r * L::kRowB + ld_slot * 16) = make_uint4(0, 0, 0, 0);
-      }
-    }
-  };
-
-  // S^T operand reads: row kt 16 + l16, piece 4 s + grp at slot (4 s + grp) ^ (l16 mod SLOTS)
-  const int k_lane = l16 * L::kRowB;
-  // V^T operand reads (transpose loads): lane (l16, grp) of the 16-lane group grp reads
-  // row 32 c + 4 grp + (l16 >> 2) (+16 for the second half) at dims 16 dt + 4 (l16 & 3),
-  // piece 2 dt + ((l16 >> 1) & 1) -> slot 2 (dt ^ m) + ((l16 >> 1) & 1), m = (l16 >> 2) & 3
-  // (^ 4 for odd grp when rows have 16 slots: the slot's bit-3 flip)
-  const int vm = ((l16 >> 2) & 3) ^ (SLOTS >= 16 ? 4 * (grp & 1) : 0);
-  const int v_lane = (4 * grp + (l16 >> 2)) * L::kRowB + ((l16 >> 1) & 1) * 16 + (l16 & 1) * 8;
-
-  float qk_scale = P.qk_scale_log2;
-  float v_mul = 1.f;
-  if (SM == 1) {
-    qk_scale *= P.k_scale[0];
-    v_mul = P.v_scale[0];
-  }
-  auto compute = [&](int tile, int b, auto full_tag) {
-    constexpr bool FULL = decltype(full_tag)::value;
-    const int base = tile * kPfKeys;
-    const uint8_t* kb = sh.k[b];
-    const uint8_t* vb = sh.v[b];
-    // per-vector scales of the lane's positions 16 kt + 4 grp + i
-    f32x4 ksv[SM == 2 ? 4 : 1], vsv[SM == 2 ? 4 : 1];
-    if constexpr (SM == 2) {
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt) {
-        ksv[kt] = *(const f32x4*)(sh.ks[b] + 16 * kt + 4 * grp);
-        vsv[kt] = *(const f32x4*)(sh.vs[b] + 16 * kt + 4 * grp);
-      }
-    }
-    // ---- S^T = K Q^T for the tile's four 16-position sub-tiles
-    f32x4 sc[4][NT];
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) sc[kt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < NQS; ++s)
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt) {
-        const uint4 a = *(const uint4*)(kb + kt * 16 * L::kRowB + k_lane +
-                                        (((4 * s + grp) ^ (l16 & (SLOTS - 1))) * 16));
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) sc[kt][nt] = M::qk(a, qreg[nt][s], sc[kt][nt]);
-      }
-    // ---- online softmax (log2 domain); lane holds positions base + 16 kt + 4 grp + i.
-    // The running max m moves only when a tile's max exceeds it by more than kPfLazy
-    // (weights stay below 2^kPfLazy), so the accumulators are rarely rescaled; the
-    // scale enters as one fma per score (qk_scale > 0: the max of raw scores scales).
-    uint4 pop[2][NT];
-    bool rescale = false;
-    float corr[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      float x[4][4];
-      float mx = -INFINITY;
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float v = sc[kt][nt][i];
-          if constexpr (SM == 2) v *= ksv[kt][i];
-          if (FULL) {
-            x[kt][i] = v;
-          } else {
-            const int pos = base + kt * 16 + 4 * grp + i;
-            x[kt][i] = (pos >= row_lo[nt] && pos < row_hi[nt]) ? v : -INFINITY;
-          }
-          mx = fmaxf(mx, x[kt][i]);
-        }
-      const float mxs = group_max(mx) * qk_scale;
-      const bool grow = mxs > m_run[nt] + kPfLazy;
-      const float m_new = grow ? mxs : m_run[nt];
-      const float m_use = m_new == -INFINITY ? 0.f : m_new;
-      corr[nt] = grow ? __builtin_amdgcn_exp2f(m_run[nt] - m_use) : 1.f;
-      rescale |= grow;
-      float rs = 0.f;
-      float pr[4][4];
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          pr[kt][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[kt][i], qk_scale, -m_use));
-          rs += pr[kt][i];
-        }
-      l_run[nt] = l_run[nt] * corr[nt] + group_sum(rs);
-      m_run[nt] = m_new;
-      if constexpr (SM == 2) {
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) pr[kt][i] *= vsv[kt][i];
-      }
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-        pop[c][nt] = make_uint4(M::pack2(pr[2 * c][0], pr[2 * c][1]),
-                                M::pack2(pr[2 * c][2], pr[2 * c][3]),
-                                M::pack2(pr[2 * c + 1][0], pr[2 * c + 1][1]),
-                                M::pack2(pr[2 * c + 1][2], pr[2 * c + 1][3]));
-    }
-    if (__builtin_amdgcn_ballot_w64(rescale) != 0) {
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int dt = 0; dt < ND; ++dt) oacc[nt][dt] *= corr[nt];
-    }
-    // ---- O^T += V^T P^T over the sub-tile pairs (2c, 2c + 1): contraction slot
-    // 8 grp + j is position 16 (2c) + 4 grp + j for j < 4, else 16 (2c + 1) + 4 grp + j - 4
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int dt = 0; dt < ND; ++dt) {
-        const uint8_t* vr = vb + 32 * c * L::kRowB + v_lane + 32 * (dt ^ vm);
-        const s16x4 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) s16x4*)(lds_void*)vr);
-        const s16x4 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) s16x4*)(lds_void*)(vr + 16 * L::kRowB));
-        uint4 a;
-        __builtin_memcpy(&a, &x0, 8);
-        __builtin_memcpy((char*)&a + 8, &x1, 8);
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) oacc[nt][dt] = M::qk(a, pop[c][nt], oacc[nt][dt]);
-      }
-  };
-
-  const int kt0 = lo_first / kPfKeys;
-  const int kt1 = (hi_last + kPfKeys - 1) / kPfKeys;
-  if (kt0 < kt1) {
-    auto step = [&](int tile, auto full_tag) {
-      const int b = (tile - kt0) & 1;
-      const bool more = tile + 1 < kt1;
-      // buffer b ^ 1 was last read in the previous iteration, before its barrier
-      if (more) load(tile + 1, b ^ 1);
-      compute(tile, b, full_tag);
-      if (more) settle(tile + 1, b ^ 1);
-      __syncthreads();
-    };
-    // tiles [fa, fb) lie inside every row's visible range: three loops, so that no
-    // branch between the two compute forms sits inside one (its join would copy the
-    // accumulators)
-    const int fa = min(kt1, max(kt0, (max(wlo, 0) + kPfKeys - 1) / kPfKeys));
-    const int fb = max(fa, min(kt1, whi / kPfKeys));
-    load(kt0, 0);
-    settle(kt0, 0);
-    __syncthreads();
-    for (int tile = kt0; tile < fa; ++tile) step(tile, Flag<false>{});
-    for (int tile = fa; tile < fb; ++tile) step(tile, Flag<true>{});
-    for (int tile = fb; tile < kt1; ++tile) step(tile, Flag<false>{});
-  }
-
-  // ---- normalized output: lane holds dims 16 dt + 4 grp + i of its rows
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int local = w * 16 * NT + nt * 16 + l16;
-    if (local >= rg_rows) continue;
-    const int rho = rg_begin + local;
-    const int qi = rho / P.group;
-    const int head = kvh * P.group + rho % P.group;
-    const int64_t off = (int64_t)(sv.q_begin + qi) * P.out_row_stride + (int64_t)head * P.out_head_stride;
-    const float inv = v_mul / fmaxf(l_run[nt], 1.0e-30f);
-#pragma unroll
-    for (int dt = 0; dt < ND; ++dt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) store_from_f32<QT>(P.out, off + dt * 16 + 4 * grp + i, oacc[nt][dt][i] * inv);
-  }
-}
+#include "prefill.h"
 
 // Window store ahead of the prefill tiling (a store-and-attend call whose window takes
 // it): one 256-thread workgroup per (64 window rows, sequence, kv head), 16 rows per
@@ -1955,14 +1527,13 @@ int launch_vec_q(const AttnParams& P, int kv_dtype, dim3 grid, hipStream_t strea
 template <int QT, int KVT, int D, int SM>
 void launch_prefill_sm(const AttnParams& P, dim3 grid, dim3 sgrid, hipStream_t stream) {
   if (P.new_k) rlt_window_store_kernel<QT, KVT, D, SM><<<sgrid, 256, 0, stream>>>(P);
-  // (fp8 pools are staged per position: the whole-tile block form is for direct loads)
-  if constexpr (KVT == QT) {
-    if (P.block_size % 16 == 0) {
-      rlt_prefill_kernel<QT, KVT, D, SM, true><<<grid, kPfThreads, 0, stream>>>(P);
-      return;
-    }
-  }
-  rlt_prefill_kernel<QT, KVT, D, SM, false><<<grid, kPfThreads, 0, stream>>>(P);
+  // blocks of whole 16-position groups, and lane offsets within a group that fit 32 bits
+  const int64_t most = (int64_t)1 << 26;
+  if (P.block_size % 16 == 0 && P.k_token_stride >= 0 && P.k_token_stride < most &&
+      P.v_token_stride >= 0 && P.v_token_stride < most)
+    rlt_prefill_kernel<QT, KVT, D, SM, true><<<grid, kPfThreads, 0, stream>>>(P);
+  else
+    rlt_prefill_kernel<QT, KVT, D, SM, false><<<grid, kPfThreads, 0, stream>>>(P);
 }
 
 template <int QT, int KVT, int D>
