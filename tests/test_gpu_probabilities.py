@@ -659,3 +659,123 @@ def test_split_form_is_batch_invariant(pkg, dev):
         idx = torch.tensor(rows, device=dev)
         small = _probs_abi(dev, logits[idx].contiguous(), t[idx], k[idx], p[idx], plan, split=True)
         assert torch.equal(small.view(torch.int32), big[idx].view(torch.int32)), rows
+
+
+# ------------------------------------------------- row-split form of filtered rows
+
+def _filter_rows(n, vocab, dtype, g):
+    """Logits whose rows the row-split filter form meets in every way: ordinary rows, one
+    dominant token (a top-k cut far below the maximum), a slice of -inf and one of the
+    type's lowest value, near-flat rows (crowded bins), ties, a temperature that scales the
+    logits out of the form's range."""
+    x = torch.randn(n, vocab, generator=g) * 3
+    t = torch.full((n,), 0.8)
+    x[1 % n, vocab // 3] += 60.0
+    x[2 % n, 8192:16384] = -torch.inf
+    x[2 % n, 16384:24576] = torch.finfo(torch.float32).min if dtype == torch.float32 else -6e4
+    x[3 % n] *= 1e-3
+    x[4 % n] = (x[4 % n] * 2).round() / 2
+    t[5 % n] = 2e-6
+    return x.to(dtype), t
+
+
+@pytest.mark.parametrize("kind", ["p", "k", "kp", "p99", "mixed"])
+@pytest.mark.parametrize("n,vocab,dtype", [
+    (8, 49153, torch.float32),     # the first vocabulary of the form, rows on odd addresses
+    (64, 57344, torch.bfloat16),   # whole slices, the most rows below 81921 columns
+    (6, 65536, torch.float16),
+    (70, 81921, torch.float32),    # one column past whole slices, more rows than 64
+    (7, 151936, torch.bfloat16),
+    (6, 262144, torch.float32),    # 32 slices
+])
+def test_filter_form_matches_exact_distributions(pkg, dev, kind, n, vocab, dtype):
+    """Filtered rows split over several workgroups against the float64 distribution and cut
+    (tolerances of the other forms' tests), on the rows of _filter_rows, at the edges of the
+    form's rule and of its slices."""
+    _say("filter form", kind, n, vocab, dtype)
+    g = torch.Generator().manual_seed(vocab + len(kind))
+    logits, t = _filter_rows(n, vocab, dtype, g)
+    i = torch.arange(n)
+    k = torch.full((n,), -1, dtype=torch.int64)
+    p = torch.ones(n)
+    if "k" in kind:
+        k = torch.tensor([50, 200, 1, 20])[i % 4]
+    if "p" in kind:
+        p = torch.full((n,), 0.99 if kind == "p99" else 0.9)
+    if kind == "mixed":
+        k = torch.tensor([-1, 40, -1, vocab - 1, 3000])[i % 5]
+        p = torch.tensor([1.0, 1.0, 0.8, 0.0])[i % 4]
+    plan = _host_args(k.tolist(), p.tolist(), vocab)
+    got = pkg.batched_probabilities(logits.to(dev), t.to(dev), k.to(dev), p.to(dev), **plan).cpu()
+    for r in sorted(set(range(min(n, 7))) | {n - 1}):
+        # the exact distribution in float64, tokens tied in x in column order
+        x = logits[r].double() / t[r].double()
+        x, order = x.sort(descending=True, stable=True)
+        at = torch.arange(vocab)
+        if plan["max_top_k"] > 0 and 0 < int(k[r]) < vocab:
+            x = x.masked_fill(at >= min(int(k[r]), plan["max_top_k"]), -torch.inf)
+        e = (x - x[0]).exp()
+        before = (e.cumsum(0) - e) / e.sum()
+        if plan["apply_top_p"] and float(p[r]) < 1:
+            kept = int((got[r] > 0).sum())
+            exact = max(1, int(((before <= float(p[r])) & (e > 0)).sum()))
+            lo, hi = min(kept, exact), max(kept, exact)
+            # the cut may lie elsewhere only where the preceding mass is within its error
+            assert ((before[lo:hi] - float(p[r])).abs() <= EXACT_BAND).all(), f"row {r}: {kept} {exact}"
+            x = x.masked_fill(at >= kept, -torch.inf)
+        want = torch.zeros(vocab, dtype=torch.float64).scatter_(0, order, x.softmax(0))
+        torch.testing.assert_close(got[r].double(), want, atol=ATOL, rtol=RTOL)
+        assert torch.equal((got[r] > 1e-30), (want > 1e-30)), f"row {r}"
+    bad = logits.clone()
+    bad[0, vocab - 1] = float("nan")
+    bad[n - 1, 0] = float("inf")
+    again = pkg.batched_probabilities(bad.to(dev), t.to(dev), k.to(dev), p.to(dev), **plan).cpu()
+    assert bool(again[0].isnan().all()) and bool(again[n - 1].isnan().all())
+    assert torch.equal(again[1:n - 1].view(torch.int32), got[1:n - 1].view(torch.int32))
+
+
+@pytest.mark.parametrize("vocab,dtype,flat", [(81921, torch.float32, False),
+                                              (98304, torch.bfloat16, True)])
+def test_filter_form_in_verify_and_draft_calls(pkg, dev, vocab, dtype, flat):
+    """The form inside the calls that use it: verify_accept equals verify_distributions and
+    speculative_accept bit for bit (row-sum partials formed from the written slices, and
+    read back for rows of the exact path), propose_drafts draws what categorical draws from
+    its q rows, argmax rows and a random row outside the logits included."""
+    _say("filter form calls", vocab, dtype, flat)
+    g = torch.Generator().manual_seed(vocab)
+    n, w1 = 3, 3
+    rows = n * (w1 + 1)
+    logits, _ = _filter_rows(rows, vocab, dtype, g)
+    if not flat:
+        logits[3] = logits[0]
+    logits = logits.to(dev)
+    t = torch.full((rows,), 0.9, device=dev)
+    k = torch.tensor([-1, 50, -1, 200]).repeat(n).to(dev)
+    p = torch.tensor([0.9, 1.0, 0.95, 0.8]).repeat(n).to(dev)
+    plan = {"max_top_k": 200, "apply_top_p": True}
+    every = torch.arange(rows, device=dev)
+    want_t, want_p = pkg.verify_distributions(logits, every, t, k, p, **plan)
+    q = torch.rand(n, w1, vocab, generator=g).to(dev)
+    q = q / q.sum(-1, keepdim=True)
+    u = torch.rand(n, w1 + 1, generator=g).to(dev)
+    draft = torch.stack([want_p[i * (w1 + 1):i * (w1 + 1) + w1].argmax(1) for i in range(n)])
+    drafts = torch.full((n,), w1, dtype=torch.int64, device=dev)
+    target, p_o, res = pkg.verify_accept(logits.view(n, w1 + 1, vocab), t, k, p, draft, drafts, q,
+                                         u[:, :w1].contiguous(), u[:, w1].contiguous(), **plan)
+    want = pkg.speculative_accept(draft, drafts, q, want_p.view(n, w1 + 1, vocab),
+                                  u[:, :w1].contiguous(), u[:, w1].contiguous())
+    assert torch.equal(target.view(-1), want_t)
+    assert torch.equal(target.view(-1).cpu(), logits.float().argmax(-1).cpu())
+    assert torch.equal(p_o.view(torch.int32), want_p.view(n, w1 + 1, vocab).view(torch.int32))
+    for a, b, name in zip(res, want, want._fields):
+        assert torch.equal(a, b), name
+    some = torch.tensor([0, 3, 4, 7, rows], device=dev)
+    ud = torch.rand(5, generator=g).to(dev)
+    pick = some.clamp(max=rows - 1)
+    proposed, q_o = pkg.propose_drafts(logits, some, t[pick], k[pick], p[pick], ud, **plan)
+    assert bool(q_o[4].isnan().all())
+    assert torch.equal(q_o[:4].view(torch.int32), want_p[some[:4]].view(torch.int32))
+    drawn = pkg.categorical(q_o[:4].contiguous(), ud[:4])[0]
+    expected = logits.float().argmax(-1)
+    expected[some[:4]] = drawn
+    assert torch.equal(proposed, expected)

@@ -270,6 +270,7 @@ __device__ __forceinline__ T wave_sum(T v) {
 }
 
 #include "probs_split.h"
+#include "probs_filter.h"
 
 template <int CAP, bool F64TOP = false, bool FAST_LANES = false>
 struct SharedT {
@@ -1293,7 +1294,7 @@ __global__ __launch_bounds__(kThreads) void rlt_probs_kernel(
       (unsigned long long)(k_eff < (int64_t)max_top_k ? k_eff : (int64_t)max_top_k);
   if (!filter_row(sh, row, dst, do_k, do_p, kk, p, z, pm_row, pm_out == nullptr)) {
     __syncthreads();
-    exact::exact_row<DT, kTC>(lds.ex, logits, src_r, row_stride, V, temperature, top_k, top_p,
+    exact::exact_row<DT, kTC>(lds.ex, r, logits, src_r, row_stride, V, temperature, top_k, top_p,
                               max_top_k, apply_top_p, out, out_stride);
   } else {
     pm_done = pm_row != nullptr;
@@ -1497,6 +1498,100 @@ void launch_split(const SplitPlan& pl, int64_t n_dist, const void* logits, const
 #undef RLT_SPLIT_E
 }
 
+// ------------------------------------------------------------------ filter form (host)
+
+// The row-split form of calls that filter (probs_filter.h): S workgroups per row.
+struct FilterPlan {
+  int S;
+};
+
+// Rows that fit on one CU (65536 columns) and are enough to fill the chip are faster there:
+// top-p 0.9 of fp32 rows, one workgroup per row against this form, 160 rows of 49152: 27 / 38
+// us, of 65536: 39 / 47, of 100001: 89 / 71, of 151936: 150 / 80; 32 rows: 24 / 24, 31 / 26, 59
+// / 33, 91 / 34; 80 rows of 65537: 38 / 35, 160: 44 / 54.
+bool filter_plan(int64_t n_dist, int V, FilterPlan& p) {
+  p.S = (V + filt::kSlice - 1) / filt::kSlice;
+  return V > 49152 && (n_dist <= 64 || V > 81920) && p.S <= filt::kMaxSlices;
+}
+
+// Its workspace: slice statistics, histograms, row cuts.
+struct FilterLayout {
+  size_t hist, cuts, total;
+  FilterLayout(const FilterPlan& pl, int64_t n_dist, int64_t n_arg) {
+    const size_t slices = (size_t)n_dist * pl.S;
+    size_t at = rlt_align_up((size_t)(n_dist + n_arg) * pl.S * sizeof(filt::SliceStat), 256);
+    auto take = [&](size_t bytes) {
+      const size_t here = at;
+      at += rlt_align_up(bytes, 256);
+      return here;
+    };
+    hist = take(slices * sizeof(filt::Hist));
+    cuts = take((size_t)n_dist * sizeof(filt::RowCut));
+    total = at;
+  }
+};
+
+size_t filter_bytes(int64_t n_dist, int64_t n_arg, int V) {
+  FilterPlan pl;
+  return n_dist > 0 && filter_plan(n_dist, V, pl) ? FilterLayout(pl, n_dist, n_arg).total : 0;
+}
+
+// Whether a filtering call takes the form: the plan, and a workspace that holds it (other
+// calls run one workgroup per row).
+bool filter_form(int64_t n_dist, int64_t n_arg, int V, const void* ws, size_t ws_bytes,
+                 FilterPlan& pl) {
+  return ws && n_dist > 0 && filter_plan(n_dist, V, pl) &&
+         ws_bytes >= FilterLayout(pl, n_dist, n_arg).total;
+}
+
+// The form's three launches (arguments as launch_split's).
+template <int DT>
+void launch_filter(const FilterPlan& pl, int64_t n_dist, const void* logits, const int64_t* rows,
+                     int64_t n_src, int64_t row_stride, int V, const filt::Filter& flt, float* out,
+                     int64_t out_stride, hipStream_t stream, int64_t* targets, int64_t n_arg,
+                     bool fused, const float* qm_src, int64_t qm_rows, float* qm_out, void* ws,
+                     float* pm_out = nullptr, double* tile_sum = nullptr,
+                     uint32_t* tile_flags = nullptr, bool skip_drawn = false) {
+  filt::View v;
+  v.S = pl.S;
+  v.n_dist = n_dist;
+  v.n_arg = fused ? 0 : n_arg;
+  const FilterLayout at(pl, n_dist, v.n_arg);
+  v.stats = (filt::SliceStat*)ws;
+  v.hist = (filt::Hist*)((char*)ws + at.hist);
+  v.cuts = (filt::RowCut*)((char*)ws + at.cuts);
+  v.targets = targets;
+  v.fused = fused;
+  v.skip_drawn = skip_drawn && rows && !fused && n_dist <= split::kMaxDrawnScan;
+  v.pm_out = pm_out;
+  v.tile_sum = tile_sum;
+  v.tile_flags = tile_flags;
+  v.tiles = (V + split::kBlockCols - 1) / split::kBlockCols;
+  const int esz = DT == RLT_F32 ? 4 : 2;
+  const bool vec = V % 4 == 0 && row_stride % 4 == 0 && (uintptr_t)logits % (4 * esz) == 0;
+  const int out_vec = out_stride % 4 == 0 && (uintptr_t)out % 16 == 0;
+  const cascade::RowGeom geo = cascade::row_geom(V);
+  const int64_t per_block = filt::kThreads / cascade::kGroupThreads;
+  const int64_t qm_blocks = qm_src ? (qm_rows * geo.groups + per_block - 1) / per_block : 0;
+  const unsigned g1 = (unsigned)((n_dist + v.n_arg) * pl.S + qm_blocks);
+  const unsigned g2 = (unsigned)(n_dist * pl.S);
+  const unsigned g3 = g2 + (unsigned)((v.n_arg + filt::kThreads - 1) / filt::kThreads);
+  const dim3 b(filt::kThreads);
+#define RLT_FILTER_LAUNCH(VEC)                                                                  \
+  filt::rlt_filter_slice_kernel<DT, VEC><<<g1, b, 0, stream>>>(                              \
+      logits, rows, n_src, row_stride, V, flt, v, qm_src, qm_rows, qm_out);                     \
+  filt::rlt_filter_row_kernel<DT, VEC><<<(unsigned)n_dist, filt::kRowThreads, 0, stream>>>(     \
+      logits, rows, n_src, row_stride, V, flt, v, out, out_stride);                             \
+  filt::rlt_filter_write_kernel<DT, VEC><<<g3, b, 0, stream>>>(                              \
+      logits, rows, n_src, row_stride, V, flt, v, out, out_stride, out_vec)
+  if (vec) {
+    RLT_FILTER_LAUNCH(true);
+  } else {
+    RLT_FILTER_LAUNCH(false);
+  }
+#undef RLT_FILTER_LAUNCH
+}
+
 }  // namespace
 
 // spec_sampling.hip: the acceptance workspace's p-row and q-row partials, and the
@@ -1532,7 +1627,9 @@ size_t rlt_probabilities_workspace_size(int64_t rows, int64_t argmax_rows, int64
   if (rows < 0 || argmax_rows < 0 || vocab < 1 || vocab > 0x7fffffff ||
       !split_plan(rows, (int)vocab, pl))
     return 0;
-  return split_bytes(rows, argmax_rows, (int)vocab);
+  const size_t sp = split_bytes(rows, argmax_rows, (int)vocab);
+  const size_t ft = filter_bytes(rows, argmax_rows, (int)vocab);
+  return sp > ft ? sp : ft;
 }
 
 int rlt_batched_probabilities(const void* logits, int32_t logits_dtype, int64_t row_stride,
@@ -1551,11 +1648,17 @@ int rlt_batched_probabilities(const void* logits, int32_t logits_dtype, int64_t 
   SplitPlan pl;
   const bool sp = workspace && mtk == 0 && !apply_top_p && split_plan(n, V, pl);
   if (sp && workspace_bytes < split_bytes(n, 0, V)) return RLT_ERR_WORKSPACE;
+  FilterPlan fl;
+  const bool ft = (mtk > 0 || apply_top_p) && filter_form(n, 0, V, workspace, workspace_bytes, fl);
+  const filt::Filter flt{temperature, top_k, top_p, mtk, apply_top_p != 0};
 #define RLT_PROBS(DT)                                                                          \
   do {                                                                                         \
     if (sp)                                                                                    \
       launch_split<DT>(pl, n, logits, nullptr, n, row_stride, V, temperature, out, out_stride, \
                        stream, nullptr, 0, false, nullptr, 0, nullptr, workspace);             \
+    else if (ft)                                                                               \
+      launch_filter<DT>(fl, n, logits, nullptr, n, row_stride, V, flt, out, out_stride, stream, \
+                        nullptr, 0, false, nullptr, 0, nullptr, workspace);                    \
     else                                                                                       \
       dispatch_probs<DT>(n, logits, nullptr, n, row_stride, V, temperature, top_k, top_p, mtk, \
                          apply_top_p != 0, out, out_stride, stream);                           \
@@ -1634,9 +1737,13 @@ int rlt_propose_drafts(const void* logits, int32_t logits_dtype, int64_t row_str
   SplitPlan pl;
   const bool sp = r > 0 && mtk == 0 && !apply_top_p && split_plan(r, V, pl) &&
                   workspace_bytes >= cat_bytes + split_bytes(r, m, V);
-  // the split form also writes the draws' tile totals (rows of at most 2M columns)
-  double* tsum = sp ? rlt_categorical_tile_sums(workspace, r, vocab) : nullptr;
-  uint32_t* tflags = sp ? rlt_categorical_tile_flags(workspace, r, vocab) : nullptr;
+  FilterPlan fl;
+  const bool ft = r > 0 && !sp && (mtk > 0 || apply_top_p) && workspace_bytes > cat_bytes &&
+                  filter_form(r, m, V, (char*)workspace + cat_bytes, workspace_bytes - cat_bytes, fl);
+  const filt::Filter flt{temperature, top_k, top_p, mtk, apply_top_p != 0};
+  // the split forms also write the draws' tile totals (rows of at most 2M columns)
+  double* tsum = sp || ft ? rlt_categorical_tile_sums(workspace, r, vocab) : nullptr;
+  uint32_t* tflags = sp || ft ? rlt_categorical_tile_flags(workspace, r, vocab) : nullptr;
   // greedy proposals for every row (extra workgroups of the distribution launch when
   // there are random rows; the split form skips the rows the draws overwrite), then
   // the random rows' draws
@@ -1649,6 +1756,10 @@ int rlt_propose_drafts(const void* logits, int32_t logits_dtype, int64_t row_str
       launch_split<DT>(pl, r, logits, random_rows, m, row_stride, V, temperature, q_out,      \
                        q_stride, stream, proposed, m, false, nullptr, 0, nullptr,             \
                        (char*)workspace + cat_bytes, nullptr, tsum, tflags, true);            \
+    else if (ft)                                                                              \
+      launch_filter<DT>(fl, r, logits, random_rows, m, row_stride, V, flt, q_out, q_stride,   \
+                        stream, proposed, m, false, nullptr, 0, nullptr,                      \
+                        (char*)workspace + cat_bytes, nullptr, tsum, tflags, true);           \
     else                                                                                      \
       dispatch_probs<DT>(r, logits, random_rows, m, row_stride, V, temperature, top_k, top_p, \
                          mtk, apply_top_p != 0, q_out, q_stride, stream, proposed, m);        \
@@ -1690,6 +1801,9 @@ int rlt_verify_distributions(const void* logits, int32_t logits_dtype, int64_t r
   SplitPlan pl;
   const bool sp = r > 0 && workspace && mtk == 0 && !apply_top_p && split_plan(r, V, pl);
   if (sp && workspace_bytes < split_bytes(r, m, V)) return RLT_ERR_WORKSPACE;
+  FilterPlan fl;
+  const bool ft = r > 0 && (mtk > 0 || apply_top_p) && filter_form(r, m, V, workspace, workspace_bytes, fl);
+  const filt::Filter flt{temperature, top_k, top_p, mtk, apply_top_p != 0};
   // targets of every row as extra workgroups of the distribution launch (split form:
   // extra slices of launch 1, finished by launch 2 or 3)
 #define RLT_VERIFY(DT)                                                                        \
@@ -1700,6 +1814,9 @@ int rlt_verify_distributions(const void* logits, int32_t logits_dtype, int64_t r
     else if (sp)                                                                              \
       launch_split<DT>(pl, r, logits, random_rows, m, row_stride, V, temperature, p_out,      \
                        p_stride, stream, targets, m, false, nullptr, 0, nullptr, workspace);  \
+    else if (ft)                                                                              \
+      launch_filter<DT>(fl, r, logits, random_rows, m, row_stride, V, flt, p_out, p_stride,   \
+                        stream, targets, m, false, nullptr, 0, nullptr, workspace);           \
     else                                                                                      \
       dispatch_probs<DT>(r, logits, random_rows, m, row_stride, V, temperature, top_k, top_p, \
                          mtk, apply_top_p != 0, p_out, p_stride, stream, targets, m);         \
@@ -1750,7 +1867,11 @@ int rlt_verify_accept(const void* target_logits, int32_t logits_dtype, int64_t r
   SplitPlan pl;
   const bool sp = mtk == 0 && !apply_top_p && split_plan(rows, V, pl, 32) &&
                   workspace_bytes >= acc_bytes + split_bytes(rows, 0, V);
-  // both forms write the p rows' row-sum partials alongside the distributions
+  FilterPlan fl;
+  const bool ft = !sp && (mtk > 0 || apply_top_p) && workspace_bytes > acc_bytes &&
+                  filter_form(rows, 0, V, (char*)workspace + acc_bytes, workspace_bytes - acc_bytes, fl);
+  const filt::Filter flt{temperature, top_k, top_p, mtk, apply_top_p != 0};
+  // every form writes the p rows' row-sum partials alongside the distributions
   float* pm_out = rlt_accept_p_partials(workspace, n, w1, vocab);
   // distributions of every verify row, their argmax targets, and the draft rows'
   // row-sum partials (one launch, or the split form's launches); then the acceptance
@@ -1761,6 +1882,10 @@ int rlt_verify_accept(const void* target_logits, int32_t logits_dtype, int64_t r
       launch_split<DT>(pl, rows, target_logits, nullptr, rows, row_stride, V, temperature,    \
                        p_out, vocab, stream, targets, rows, true, q_rows > 0 ? q : nullptr,   \
                        q_rows, qm_out, (char*)workspace + acc_bytes, pm_out);                 \
+    else if (ft)                                                                              \
+      launch_filter<DT>(fl, rows, target_logits, nullptr, rows, row_stride, V, flt, p_out,    \
+                        vocab, stream, targets, rows, true, q_rows > 0 ? q : nullptr, q_rows, \
+                        qm_out, (char*)workspace + acc_bytes, pm_out);                        \
     else                                                                                      \
       dispatch_probs<DT>(rows, target_logits, nullptr, rows, row_stride, V, temperature,      \
                          top_k, top_p, mtk, apply_top_p != 0, p_out, vocab, stream, targets,  \

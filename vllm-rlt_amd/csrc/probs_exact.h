@@ -360,11 +360,11 @@ __device__ __forceinline__ Cut select_cut(Shared& sh, const R& row, float m,
   return c;
 }
 
-// One row (block r = blockIdx.x, logits row src_r) on the re-reading variant; sh is
-// the caller's LDS.
+// Output row r (logits row src_r) on the re-reading variant; sh is the caller's LDS.
 template <int DT, int TC>
-__device__ __forceinline__ void exact_row(SharedT<TC>& sh, const void* __restrict__ logits,
-                                          int64_t src_r, int64_t row_stride, int V,
+__device__ __forceinline__ void exact_row(SharedT<TC>& sh, int64_t r,
+                                          const void* __restrict__ logits, int64_t src_r,
+                                          int64_t row_stride, int V,
                                           const float* __restrict__ temperature,
                                           const int64_t* __restrict__ top_k,
                                           const float* __restrict__ top_p, int max_top_k,
@@ -374,7 +374,6 @@ __device__ __forceinline__ void exact_row(SharedT<TC>& sh, const void* __restric
   (void)NREG;
   (void)NLDS;
   float* const xlds = nullptr;
-  const int64_t r = blockIdx.x;
   const int t = threadIdx.x, w = t >> 6, lane = t & 63;
   Row<DT, NREG, NLDS> row;
   row.xl = xlds;
