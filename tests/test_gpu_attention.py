@@ -1132,3 +1132,50 @@ def test_packed_window_shape_selects_compensation(pkg, dev):
     assert not pkg.create_backend("auto", dev, torch.bfloat16, 128, 16).kernel.compensate
     assert not pkg.create_backend("auto", dev, torch.float16, 128, 16,
                                   packed_window_shape=shape).kernel.compensate
+
+
+@pytest.mark.parametrize("kv", ["same", "fp8", "fp8_vector"])
+@pytest.mark.parametrize("d,hkv", [(64, 1), (96, 3), (128, 2), (128, 8)])
+def test_long_window_store_ragged_rows(kernel, pkg, dev, kv, d, hkv):
+    """The window store ahead of the prefill tiling on ragged windows (none, one row, a
+    window that starts at position 0, one past a workgroup's vectors): exactly the bits of
+    store_kv / store_fp8, and no other byte of the pool touched."""
+    _say("ragged window store", kv, d, hkv)
+    g = torch.Generator().manual_seed(d + hkv)
+    dtype, bs, q_lens = torch.bfloat16, 16, [64, 0, 1, 33, 131, 70]
+    lengths = [64, 40, 7, 2049, 500, 513]
+    pages = sum(-(-x // bs) for x in lengths) + 4
+    tables = random_tables(lengths, bs, pages, g)
+    rows = sum(q_lens)
+    q = torch.randn(rows, 2 * hkv, d, generator=g).to(dtype).to(dev)
+    k_new, v_new = ((torch.randn(rows, hkv, d, generator=g) * 4).to(dtype).to(dev)
+                    for _ in range(2))
+    seq = torch.repeat_interleave(torch.arange(len(q_lens)), torch.tensor(q_lens))
+    pos = torch.cat([torch.arange(c - w, c) for c, w in zip(lengths, q_lens)])
+    blocks, offs = tables.long()[seq, pos // bs].to(dev), (pos % bs).to(dev)
+    shape = (pages, bs, hkv, d)
+    scales = None
+    if kv == "same":
+        pools = [torch.randn(shape, generator=g).to(dtype).to(dev) for _ in range(2)]
+    else:
+        pools = [torch.randint(0, 120, shape, generator=g, dtype=torch.uint8).to(dev).view(
+            torch.float8_e4m3fn) for _ in range(2)]
+        scales = [torch.full(shape[:-1], 0.5, device=dev) for _ in range(2)]
+    want = [x.clone() for x in pools]
+    want_scales = [x.clone() for x in scales] if scales else None
+    if kv == "same":
+        pkg.store_kv(*want, k_new, v_new, blocks, offs)
+        args = ()
+    else:
+        pkg.store_fp8(k_new, v_new, *want, *want_scales, blocks, offs, 448.0,
+                      fixed_scale=0.0375 if kv == "fp8" else None)
+        args = tuple(scales) if kv == "fp8_vector" else (torch.tensor(0.0375, device=dev),) * 2
+    cu = torch.tensor([0] + torch.cumsum(torch.tensor(q_lens), 0).tolist(), dtype=torch.int32)
+    assert kernel.uses_prefill_tiling(dtype, pools[0].dtype, d, max(q_lens))
+    kernel.prefill_store(q, k_new, v_new, *pools, tables.to(dev),
+                         torch.tensor(lengths, dtype=torch.int32).to(dev), cu.to(dev),
+                         max(q_lens), *args)
+    for got, ref in zip(pools, want):
+        assert torch.equal(got.view(torch.uint8), ref.view(torch.uint8))
+    if kv == "fp8_vector":
+        assert all(torch.equal(a, b) for a, b in zip(scales, want_scales))

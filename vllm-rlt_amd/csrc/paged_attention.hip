@@ -1443,18 +1443,115 @@ __global__ __launch_bounds__(256) void rlt_merge_kernel(AttnParams P) {
 #include "prefill.h"
 
 // Window store ahead of the prefill tiling (a store-and-attend call whose window takes
-// it): one 256-thread workgroup per (64 window rows, sequence, kv head), 16 rows per
-// wave, the verify kernels' fused per-row stores (store_rows).
+// it).  A group of 8 or 16 lanes takes one vector -- a window row's key or value of one kv
+// head, 16 bytes a lane -- and a workgroup kStoreVectors consecutive vectors of a sequence
+// (kv heads innermost, keys before values), with the loads of all of a lane's vectors in
+// flight before the first is quantized.  The bits are store_rows' (the verify kernels'
+// fused store).
+//
+// What bounds it: memory latency on short chunks, then HBM.  A wave that took 16 rows of a
+// kv head one after the other waited for a row's load, its table entry and its reduction
+// 16 times over: 2820 rows of 8 heads, D = 128, quantized with per-vector scales 37.9 us,
+// here 15.3; 8 x 2048 rows of 4 heads in bf16, 13.9.
+constexpr int kStoreThreads = 256;
+constexpr int kStoreDepth = 4;  // vectors per lane group
+template <int D>
+constexpr int store_lanes() { return D <= 64 ? 8 : 16; }
+template <int D>
+constexpr int store_vectors() { return kStoreThreads / store_lanes<D>() * kStoreDepth; }
+
+// NaN-propagating maximum over a group of L (8 or 16) lanes, in every lane.
+template <int L>
+__device__ __forceinline__ float group_nan_max(float x) {
+  auto at = [](float v, auto ctrl) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value,
+                                                      0xf, 0xf, false));
+  };
+  x = rlt_fp8::nan_max(x, at(x, std::integral_constant<int, 0xB1>{}));   // lane ^ 1
+  x = rlt_fp8::nan_max(x, at(x, std::integral_constant<int, 0x4E>{}));   // lane ^ 2
+  x = rlt_fp8::nan_max(x, at(x, std::integral_constant<int, 0x141>{}));  // 8 lanes mirrored
+  if (L == 16) x = rlt_fp8::nan_max(x, at(x, std::integral_constant<int, 0x140>{}));
+  return x;
+}
+
 template <int QT, int KVT, int D, int SM>
-__global__ __launch_bounds__(256) void rlt_window_store_kernel(AttnParams P) {
-  const int64_t id = blockIdx.x;
-  const int kvh = (int)(id % P.hkv);
-  const int64_t sr = id / P.hkv;
-  const int seq = (int)(sr % P.num_seqs);
-  const int i0 = (int)(sr / P.num_seqs) * 64 + (int)(threadIdx.x >> 6) * 16;
+__global__ __launch_bounds__(kStoreThreads) void rlt_window_store_kernel(AttnParams P, int per_seq) {
+  constexpr int LPV = store_lanes<D>();
+  constexpr int kPieces = D / 8;  // 16-byte pieces of a vector
+  constexpr int kAtOnce = kStoreThreads / LPV;
+  const int seq = (int)(blockIdx.x / (unsigned)per_seq);
+  const int64_t first = (int64_t)(blockIdx.x - (unsigned)seq * per_seq) * store_vectors<D>();
   const SeqView sv = seq_view(P, seq);
-  if (i0 >= sv.q_len) return;  // wave-uniform; no barriers follow
-  store_rows<QT, KVT, D, SM>(P, seq, kvh, sv, i0, min(sv.q_len, i0 + 16), 0, INT_MAX);
+  const uint32_t vectors = 2 * P.hkv;  // of one row
+  const int row0 = (int)(first / vectors);
+  if (row0 >= sv.q_len) return;
+  const uint32_t off0 = (uint32_t)(first - (int64_t)row0 * vectors);
+  const int sub = threadIdx.x / LPV, piece = threadIdx.x % LPV;
+  uint4 raw[kStoreDepth];
+  int32_t entry[kStoreDepth];
+  int head[kStoreDepth], off[kStoreDepth];
+  bool value[kStoreDepth];
+#pragma unroll
+  for (int u = 0; u < kStoreDepth; ++u) {
+    const uint32_t at = off0 + sub + u * kAtOnce;
+    const int i = row0 + (int)(at / vectors);
+    const uint32_t vec = at % vectors;
+    value[u] = vec >= (uint32_t)P.hkv;
+    head[u] = (int)(value[u] ? vec - P.hkv : vec);
+    // positions before the sequence, past the block table or outside the pool are not
+    // written
+    const int pos = sv.kv_len - sv.q_len + i;
+    const int idx = pos / P.block_size;
+    off[u] = pos % P.block_size;
+    const bool live = i < sv.q_len && pos >= 0 && idx < P.table_width;
+    entry[u] = live ? P.tables[(int64_t)seq * P.table_stride + idx] : -1;
+    raw[u] = make_uint4(0, 0, 0, 0);
+    if (live && piece < kPieces)
+      raw[u] = ((const uint4*)((const uint16_t*)(value[u] ? P.new_v : P.new_k) +
+                               (int64_t)(sv.q_begin + i) * P.new_row_stride +
+                               (int64_t)head[u] * P.new_head_stride))[piece];
+  }
+#pragma unroll
+  for (int u = 0; u < kStoreDepth; ++u) {
+    const bool store = entry[u] >= 0 && entry[u] < P.num_blocks;
+    const int64_t at = (int64_t)entry[u] * (value[u] ? P.v_block_stride : P.k_block_stride) +
+                       (int64_t)off[u] * (value[u] ? P.v_token_stride : P.k_token_stride) +
+                       (int64_t)head[u] * (value[u] ? P.v_head_stride : P.k_head_stride);
+    uint8_t* pool = (uint8_t*)(value[u] ? P.v : P.k);
+    if constexpr (KVT == QT) {
+      if (store && piece < kPieces) ((uint4*)(pool + 2 * at))[piece] = raw[u];
+    } else {
+      const uint32_t w4[4] = {raw[u].x, raw[u].y, raw[u].z, raw[u].w};
+      float x[8];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        x[2 * j] = Mfma<QT>::lo_f32(w4[j]);
+        x[2 * j + 1] = Mfma<QT>::hi_f32(w4[j]);
+      }
+      float* scales = const_cast<float*>(value[u] ? P.v_scale : P.k_scale);
+      float scale;
+      if constexpr (SM == 2) {
+        float amax = 0.f;  // (lanes past the vector hold zeros)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) amax = rlt_fp8::nan_max(amax, fabsf(x[j]));
+        scale = rlt_fp8::dynamic_scale(group_nan_max<LPV>(amax));
+      } else {
+        scale = scales[0];
+      }
+      if (store && piece < kPieces) {
+        uint32_t lo = 0, hi = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          lo |= rlt_fp8::encode(x[j], scale) << (8 * j);
+          hi |= rlt_fp8::encode(x[4 + j], scale) << (8 * j);
+        }
+        *(uint2*)(pool + at + 8 * piece) = make_uint2(lo, hi);
+        if (SM == 2 && piece == 0)
+          scales[(int64_t)entry[u] * P.s_block_stride + (int64_t)off[u] * P.s_token_stride +
+                 (int64_t)head[u] * P.s_head_stride] = scale;
+      }
+    }
+  }
 }
 
 // ============================================================ dispatch
@@ -1525,8 +1622,13 @@ int launch_vec_q(const AttnParams& P, int kv_dtype, dim3 grid, hipStream_t strea
 }
 
 template <int QT, int KVT, int D, int SM>
-void launch_prefill_sm(const AttnParams& P, dim3 grid, dim3 sgrid, hipStream_t stream) {
-  if (P.new_k) rlt_window_store_kernel<QT, KVT, D, SM><<<sgrid, 256, 0, stream>>>(P);
+void launch_prefill_sm(const AttnParams& P, dim3 grid, int max_q, hipStream_t stream) {
+  if (P.new_k) {
+    // (attention_impl bounds the product)
+    const int64_t per_seq = ((int64_t)max_q * 2 * P.hkv + store_vectors<D>() - 1) / store_vectors<D>();
+    rlt_window_store_kernel<QT, KVT, D, SM><<<(unsigned)(P.num_seqs * per_seq), kStoreThreads, 0, stream>>>(
+        P, (int)per_seq);
+  }
   // blocks of whole 16-position groups, and lane offsets within a group that fit 32 bits
   const int64_t most = (int64_t)1 << 26;
   if (P.block_size % 16 == 0 && P.k_token_stride >= 0 && P.k_token_stride < most &&
@@ -1537,18 +1639,18 @@ void launch_prefill_sm(const AttnParams& P, dim3 grid, dim3 sgrid, hipStream_t s
 }
 
 template <int QT, int KVT, int D>
-void launch_prefill_d(const AttnParams& P, dim3 grid, dim3 sgrid, hipStream_t stream) {
-  if constexpr (KVT == QT) launch_prefill_sm<QT, KVT, D, 0>(P, grid, sgrid, stream);
-  else if (P.scale_mode == 1) launch_prefill_sm<QT, KVT, D, 1>(P, grid, sgrid, stream);
-  else launch_prefill_sm<QT, KVT, D, 2>(P, grid, sgrid, stream);
+void launch_prefill_d(const AttnParams& P, dim3 grid, int max_q, hipStream_t stream) {
+  if constexpr (KVT == QT) launch_prefill_sm<QT, KVT, D, 0>(P, grid, max_q, stream);
+  else if (P.scale_mode == 1) launch_prefill_sm<QT, KVT, D, 1>(P, grid, max_q, stream);
+  else launch_prefill_sm<QT, KVT, D, 2>(P, grid, max_q, stream);
 }
 
-// sgrid: the window store's grid (launched first when the call stores its rows)
+// max_q: the longest window (the store of the rows, when the call has one, goes first)
 template <int QT, int KVT>
-void launch_prefill(const AttnParams& P, int head_dim, dim3 grid, dim3 sgrid, hipStream_t stream) {
-  if (head_dim == 64) launch_prefill_d<QT, KVT, 64>(P, grid, sgrid, stream);
-  else if (head_dim == 96) launch_prefill_d<QT, KVT, 96>(P, grid, sgrid, stream);
-  else launch_prefill_d<QT, KVT, 128>(P, grid, sgrid, stream);
+void launch_prefill(const AttnParams& P, int head_dim, dim3 grid, int max_q, hipStream_t stream) {
+  if (head_dim == 64) launch_prefill_d<QT, KVT, 64>(P, grid, max_q, stream);
+  else if (head_dim == 96) launch_prefill_d<QT, KVT, 96>(P, grid, max_q, stream);
+  else launch_prefill_d<QT, KVT, 128>(P, grid, max_q, stream);
 }
 
 template <int OT>
@@ -1738,16 +1840,16 @@ int attention_impl(const void* q, int64_t q_row_stride, int64_t q_head_stride,
       const int64_t wgs = (int64_t)num_seqs * P.rowgroups * num_kv_heads;
       if (wgs >= ((int64_t)1 << 31)) return RLT_ERR_UNSUPPORTED;
       const dim3 grid((unsigned)wgs);
-      const int64_t swgs = (int64_t)num_seqs * num_kv_heads * ((max_q_len + 63) / 64);
+      // the window store's workgroups (at least 64 vectors each, two per row and kv head)
+      const int64_t swgs = (int64_t)num_seqs * num_kv_heads * (((int64_t)max_q_len + 31) / 32);
       if (swgs >= ((int64_t)1 << 31)) return RLT_ERR_UNSUPPORTED;
-      const dim3 sgrid((unsigned)swgs);
       const bool fp8 = kv_dtype == RLT_FP8_E4M3;
       if (q_dtype == RLT_BF16) {
-        if (fp8) launch_prefill<RLT_BF16, RLT_FP8_E4M3>(P, head_dim, grid, sgrid, stream);
-        else launch_prefill<RLT_BF16, RLT_BF16>(P, head_dim, grid, sgrid, stream);
+        if (fp8) launch_prefill<RLT_BF16, RLT_FP8_E4M3>(P, head_dim, grid, max_q_len, stream);
+        else launch_prefill<RLT_BF16, RLT_BF16>(P, head_dim, grid, max_q_len, stream);
       } else {
-        if (fp8) launch_prefill<RLT_F16, RLT_FP8_E4M3>(P, head_dim, grid, sgrid, stream);
-        else launch_prefill<RLT_F16, RLT_F16>(P, head_dim, grid, sgrid, stream);
+        if (fp8) launch_prefill<RLT_F16, RLT_FP8_E4M3>(P, head_dim, grid, max_q_len, stream);
+        else launch_prefill<RLT_F16, RLT_F16>(P, head_dim, grid, max_q_len, stream);
       }
       return rlt_launch_status();
     }
