@@ -12,8 +12,8 @@
 // Work decomposition (static grids, graph-capturable: no host-side length reads):
 //  The unit of work is (sequence x row-group, kv head, chunk), a chunk being
 //  512 absolute key positions [512c, 512c + 512) (1024 for fp8 KV on the MFMA path)
-//  processed in 16-position tiles by two waves (one for fp8 KV) whose states combine
-//  in a fixed order.  Every row of the sequence (q_len window rows x GQA group)
+//  processed in pairs of 16-position tiles by two waves (one for fp8 KV) whose states
+//  combine in a fixed order.  Every row of the sequence (q_len window rows x GQA group)
 //  that attends to the kv head is in the unit's row-group, so each KV byte is read
 //  once per (sequence, kv head) instead of once per q row.  On the MFMA path one
 //  persistent 8-wave workgroup per CU enumerates the active units from the
@@ -35,9 +35,14 @@
 //    S^T = K Q^T with v_mfma_f32_16x16x32_{bf16,f16} straight from global memory
 //    (the contraction order is permuted so that each lane's eight elements per
 //    step are contiguous in memory: the A-operand layout), online softmax in fp32
-//    (log2 domain), then O^T = V^T P^T with v_mfma_f32_16x16x16: the P^T operand
-//    is exactly the S^T accumulator layout, and the output dimensions are permuted
-//    so that V^T operands are contiguous loads too (no LDS transpose).
+//    (log2 domain), then O^T = V^T P^T with the same instruction over a pair of
+//    tiles: the P^T operand is the pair's S^T accumulators as they lie (the contraction
+//    order is free), and the output dimensions are permuted so that V^T operands are
+//    contiguous loads too (no LDS transpose).  A pair at a time because the step is a
+//    serial chain -- scores, maximum over lanes, exponentials, sum over lanes, products --
+//    that a wave alone on its SIMD waits through (0.48 us per 16 positions before).  One
+//    row at 700 positions, 16 heads: 17.4 -> 15.6 us; 8 rows of fp8 at 2-4k: 49 -> 38;
+//    windows of 5 at up to 8k: 80.8 -> 79.0; 64 x 4 planes of fp8 at 16-32k: 2.51 -> 2.43 ms.
 //  * vector (fp32 q, or any other head_dim <= 256): fp32 FMA dot products.
 
 #include "common.h"
@@ -55,7 +60,6 @@ constexpr int kChunk = 512;       // key positions per workgroup (split unit)
 constexpr int kWaves = 4;
 constexpr int kWaveSpan = kChunk / kWaves;  // 128 positions per wave
 constexpr int kTileTok = 16;
-constexpr int kStages = 2;  // KV tiles in flight per wave (MFMA path)
 // Waves per work unit on the MFMA path (equal position spans combined in a fixed
 // order): two for 16-bit KV; one for fp8 KV, whose 512-position unit is half the bytes
 // (one wave streams it alone faster than two that wait at the combine).  Fixed per
@@ -221,7 +225,6 @@ __device__ __forceinline__ void merge_scales(float m1, float m2, float& mo, floa
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 template <int QT>
@@ -229,17 +232,11 @@ struct Mfma;
 
 template <>
 struct Mfma<RLT_BF16> {
-  __device__ static f32x4 qk(uint4 a, uint4 b, f32x4 c) {
+  __device__ static f32x4 mma(uint4 a, uint4 b, f32x4 c) {
     bf16x8 av, bv;
     __builtin_memcpy(&av, &a, 16);
     __builtin_memcpy(&bv, &b, 16);
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, c, 0, 0, 0);
-  }
-  __device__ static f32x4 pv(uint2 a, uint2 b, f32x4 c) {
-    s16x4 av, bv;
-    __builtin_memcpy(&av, &a, 8);
-    __builtin_memcpy(&bv, &b, 8);
-    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, c, 0, 0, 0);
   }
   __device__ static uint16_t from_f32(float x) { return f32_to_bf16_bits(x); }
   // the two values of a packed pair, exactly
@@ -255,17 +252,11 @@ struct Mfma<RLT_BF16> {
 
 template <>
 struct Mfma<RLT_F16> {
-  __device__ static f32x4 qk(uint4 a, uint4 b, f32x4 c) {
+  __device__ static f32x4 mma(uint4 a, uint4 b, f32x4 c) {
     f16x8 av, bv;
     __builtin_memcpy(&av, &a, 16);
     __builtin_memcpy(&bv, &b, 16);
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bv, c, 0, 0, 0);
-  }
-  __device__ static f32x4 pv(uint2 a, uint2 b, f32x4 c) {
-    f16x4 av, bv;
-    __builtin_memcpy(&av, &a, 8);
-    __builtin_memcpy(&bv, &b, 8);
-    return __builtin_amdgcn_mfma_f32_16x16x16f16(av, bv, c, 0, 0, 0);
   }
   __device__ static uint16_t from_f32(float x) { return f32_to_f16_bits(x); }
   __device__ static float lo_f32(uint32_t w) { return f16_bits_to_f32((uint16_t)(w & 0xffffu)); }
@@ -282,17 +273,18 @@ struct Flag {
   static constexpr bool value = B;
 };
 
-// Four fp8 codes -> four 16-bit values of the MFMA type (exact for e4m3; two gfx950
-// pair conversions, where the way through fp32 took four and the packing).
+// Two fp8 codes (the low or high half of w) -> packed 16-bit values of the MFMA type
+// (exact for e4m3; one gfx950 pair conversion).
+template <int QT, bool kHigh>
+__device__ __forceinline__ uint32_t fp8x2_to_16(uint32_t w) {
+  if (QT == RLT_BF16)
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.f, kHigh));
+  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.f, kHigh));
+}
+// Four codes -> four values.
 template <int QT>
 __device__ __forceinline__ uint2 fp8x4_to_16(uint32_t w) {
-  if (QT == RLT_BF16)
-    return make_uint2(
-        __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.f, false)),
-        __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.f, true)));
-  return make_uint2(
-      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.f, false)),
-      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.f, true)));
+  return make_uint2(fp8x2_to_16<QT, false>(w), fp8x2_to_16<QT, true>(w));
 }
 
 // One lane's raw key elements, as loaded from HBM: for contraction step s the
@@ -339,9 +331,8 @@ struct RawSlice {
       }
     }
   }
-  // The eight elements of step s as MFMA operand bits;
-  // zeros when `ok` is false (positions past the sequence may hold any bits).
-  __device__ __forceinline__ uint4 op(int s, bool ok) const {
+  // The eight elements of step s as MFMA operand bits.
+  __device__ __forceinline__ uint4 op(int s) const {
     uint4 r;
     if (KVT == QT) {
       r = make_uint4(w[4 * s], w[4 * s + 1], w[4 * s + 2], w[4 * s + 3]);
@@ -350,7 +341,6 @@ struct RawSlice {
       const uint2 b = fp8x4_to_16<QT>(w[2 * s + 1]);
       r = make_uint4(a.x, a.y, b.x, b.y);
     }
-    if (!ok) r = make_uint4(0, 0, 0, 0);
     return r;
   }
 };
@@ -405,24 +395,15 @@ struct ValueQuad {
       a0.y = __builtin_amdgcn_perm(w[3][K], w[2][K], 0x05040100u);
       a1.y = __builtin_amdgcn_perm(w[3][K], w[2][K], 0x07060302u);
     } else {
-      float2 f[4];
+      // dims 2k and 2k + 1 of each position widened (exact for e4m3), then as above
+      uint32_t f[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (kHalfWords) f[i] = fp8x2_to_f32<false>(w[i][K]);
-        else f[i] = (K & 1) ? fp8x2_to_f32<true>(w[i][K / 2]) : fp8x2_to_f32<false>(w[i][K / 2]);
-      }
-      if (QT == RLT_BF16) {
-        // e4m3 values are exact in bf16: the high half of the fp32 bits
-        a0.x = __builtin_amdgcn_perm(__float_as_uint(f[1].x), __float_as_uint(f[0].x), 0x07060302u);
-        a1.x = __builtin_amdgcn_perm(__float_as_uint(f[1].y), __float_as_uint(f[0].y), 0x07060302u);
-        a0.y = __builtin_amdgcn_perm(__float_as_uint(f[3].x), __float_as_uint(f[2].x), 0x07060302u);
-        a1.y = __builtin_amdgcn_perm(__float_as_uint(f[3].y), __float_as_uint(f[2].y), 0x07060302u);
-      } else {
-        a0.x = (uint32_t)f32_to_f16_bits(f[0].x) | ((uint32_t)f32_to_f16_bits(f[1].x) << 16);
-        a1.x = (uint32_t)f32_to_f16_bits(f[0].y) | ((uint32_t)f32_to_f16_bits(f[1].y) << 16);
-        a0.y = (uint32_t)f32_to_f16_bits(f[2].x) | ((uint32_t)f32_to_f16_bits(f[3].x) << 16);
-        a1.y = (uint32_t)f32_to_f16_bits(f[2].y) | ((uint32_t)f32_to_f16_bits(f[3].y) << 16);
-      }
+      for (int i = 0; i < 4; ++i)
+        f[i] = kHalfWords ? fp8x2_to_16<QT, false>(w[i][K]) : fp8x2_to_16<QT, (K & 1) != 0>(w[i][K / 2]);
+      a0.x = __builtin_amdgcn_perm(f[1], f[0], 0x05040100u);
+      a1.x = __builtin_amdgcn_perm(f[1], f[0], 0x07060302u);
+      a0.y = __builtin_amdgcn_perm(f[3], f[2], 0x05040100u);
+      a1.y = __builtin_amdgcn_perm(f[3], f[2], 0x07060302u);
     }
   }
 };
@@ -595,6 +576,12 @@ __device__ __forceinline__ void attend_span(const AttnParams& P, int seq, int rg
   const int lane = threadIdx.x & 63;
   const int l16 = lane & 15;
   const int grp = lane >> 4;
+  // (the same in every lane of the wave: scalar registers and scalar loads)
+  seq = __builtin_amdgcn_readfirstlane(seq);
+  rg = __builtin_amdgcn_readfirstlane(rg);
+  kvh = __builtin_amdgcn_readfirstlane(kvh);
+  chunk = __builtin_amdgcn_readfirstlane(chunk);
+  part = __builtin_amdgcn_readfirstlane(part);
   const int c_begin = chunk * CH;
   const int w_begin = c_begin + part * kSpan;
 
@@ -684,176 +671,228 @@ __device__ __forceinline__ void attend_span(const AttnParams& P, int seq, int rg
   }
 
   if (t0 < t1) {
-    Raw kb[kStages];
-    VQ vq[kStages];
-    float ksc[kStages][4], vsc[kStages][4];
-    bool okk[kStages];
-    uint32_t okv[kStages];  // bit i: value position 4 * grp + i is inside the sequence
+    // Two tiles (a pair, 32 absolute positions) at a time: one softmax step and 32-wide
+    // contractions over both.
+    // (256 16-bit dims: the second tile's keys wait until the products are done, the
+    // registers do not hold both pairs)
+    constexpr bool kLateKey = D > 128 && KV_ELT == 2;
+    Raw kb[2];
+    VQ vq[2];
+    float sraw = 0.f;
     const int64_t k_head = (int64_t)kvh * P.k_head_stride + grp * Raw::kGroupElems;
     const int64_t v_head = (int64_t)kvh * P.v_head_stride + l16 * ND;
     const int32_t* tbl = tbl_lds - c_begin;  // tbl[pos] for pos in the chunk
-    // Loads of tile t into stage b.  Branch-free: every address is inside the
-    // pool, and positions outside the sequence are zeroed at use.
-    auto issue = [&](int t, int b) {
-      const int tb = w_begin + t * kTileTok;
-      okk[b] = tb + l16 < hi_last;
-      uint32_t m4 = 0;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) m4 |= (tb + 4 * grp + i < hi_last) ? (1u << i) : 0u;
-      okv[b] = m4;
+    // positions of the span's tiles: [read_lo, hi_last); the others of a pair are masked,
+    // their values taken as zeros (they may hold any bits, NaN included)
+    const int read_lo = w_begin + t0 * kTileTok;
+    auto inside = [&](int pos) { return pos >= read_lo && pos < hi_last; };
+    // Loads of tile t into half b of the pair.  Branch-free: the tile is clamped into the
+    // span's tiles, so every address is one that some row reads.
+    const int tl = t1 - 1;
+    auto tile_base = [&](int t) { return w_begin + min(max(t, t0), tl) * kTileTok; };
+    // With whole tiles per block the block is wave-uniform: a scalar base and a 32-bit lane
+    // offset (fewer address registers; launch_mfma_sm bounds the strides).
+    const uint32_t k_lane = (uint32_t)(l16 * (uint32_t)P.k_token_stride + grp * Raw::kGroupElems) * KV_ELT;
+    const uint32_t v_lane = (uint32_t)(4 * grp * (uint32_t)P.v_token_stride + l16 * ND) * KV_ELT;
+    auto issue_k = [&](int t, int b) {
+      const int tb = tile_base(t);
       if (UB) {
         const int64_t bk = __builtin_amdgcn_readfirstlane(tbl[tb]);
-        const int in_blk = tb % P.block_size;
-        const uint8_t* kp = (const uint8_t*)P.k +
-            (bk * P.k_block_stride + (int64_t)(in_blk + l16) * P.k_token_stride + k_head) * KV_ELT;
-        kb[b].load(kp);
-        const uint8_t* vbase = (const uint8_t*)P.v + (bk * P.v_block_stride + v_head) * KV_ELT;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          vq[b].load(i, vbase + (int64_t)(in_blk + 4 * grp + i) * P.v_token_stride * KV_ELT);
+        const uint8_t* base = (const uint8_t*)P.k +
+            (bk * P.k_block_stride + (int64_t)(tb % P.block_size) * P.k_token_stride +
+             (int64_t)kvh * P.k_head_stride) * KV_ELT;
+        kb[b].load(base + k_lane);
       } else {
         const int64_t bk = tbl[tb + l16];
-        const uint8_t* kp = (const uint8_t*)P.k +
-            (bk * P.k_block_stride + (int64_t)((tb + l16) % P.block_size) * P.k_token_stride + k_head) *
-                KV_ELT;
-        kb[b].load(kp);
+        kb[b].load((const uint8_t*)P.k +
+                   (bk * P.k_block_stride + (int64_t)((tb + l16) % P.block_size) * P.k_token_stride + k_head) *
+                       KV_ELT);
+      }
+    };
+    auto issue_v = [&](int t, int b) {
+      const int tb = tile_base(t);
+      if (UB) {
+        const int64_t bk = __builtin_amdgcn_readfirstlane(tbl[tb]);
+        const uint8_t* base = (const uint8_t*)P.v +
+            (bk * P.v_block_stride + (int64_t)(tb % P.block_size) * P.v_token_stride +
+             (int64_t)kvh * P.v_head_stride) * KV_ELT;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vq[b].load(i, base + (int64_t)i * P.v_token_stride * KV_ELT + v_lane);
+      } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int pv = tb + 4 * grp + i;
           const int64_t bv = tbl[pv];
-          const uint8_t* vp = (const uint8_t*)P.v +
-              (bv * P.v_block_stride + (int64_t)(pv % P.block_size) * P.v_token_stride + v_head) * KV_ELT;
-          vq[b].load(i, vp);
-        }
-      }
-      if (SM == 2) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int p4 = tb + 4 * grp + r;
-          // with whole tiles per block only the tile's first entry is stored
-          const int64_t so = (int64_t)tbl[UB ? tb : p4] * P.s_block_stride +
-                             (int64_t)(p4 % P.block_size) * P.s_token_stride +
-                             (int64_t)kvh * P.s_head_stride;
-          const bool ok4 = p4 < hi_last;
-          ksc[b][r] = ok4 ? P.k_scale[so] : 0.f;
-          vsc[b][r] = ok4 ? P.v_scale[so] : 0.f;
+          vq[b].load(i, (const uint8_t*)P.v +
+              (bv * P.v_block_stride + (int64_t)(pv % P.block_size) * P.v_token_stride + v_head) * KV_ELT);
         }
       }
     };
-    // Wave-uniform fast-path bound: a tile inside [lo of the last row, hi of the
+    // Per-vector scales, one load a lane: lane group 0 takes the key scales of tile t, 1 of
+    // tile t + 1, 2 and 3 the value scales, each lane one position; lanes fetch the scales of
+    // their accumulator rows from them at use (a load per position and lane group was more
+    // load instructions than the keys and values: 8 windows of 5 at 2-4k, 8 kv heads, 67.8
+    // -> 52.9 us).
+    auto issue_scales = [&](int t) {
+      if (SM == 2) {
+        const int tb = (grp & 1) ? tile_base(t + 1) : tile_base(t);
+        const int64_t so = (int64_t)tbl[UB ? tb : tb + l16] * P.s_block_stride +
+                           (int64_t)((tb + l16) % P.block_size) * P.s_token_stride +
+                           (int64_t)kvh * P.s_head_stride;
+        sraw = (grp < 2 ? P.k_scale : P.v_scale)[so];
+      }
+    };
+    auto scale_of = [&](float x, int b, int r) {
+      return __int_as_float(__builtin_amdgcn_ds_bpermute(16 * grp + 64 * b + 4 * r, __float_as_int(x)));
+    };
+    // Wave-uniform fast-path bound: a pair inside [lo of the last row, hi of the
     // first row) is visible to every row of the row-group and fully stored, so
-    // it needs no position masks.  Both paths compute identical bits for a row.
-    const int full_lo = lo_last;
+    // it needs no position masks.  (Branches around the masks: two copies of the whole
+    // step, one without them, cost registers that D = 256 and two row tiles do not have.)
+    const int full_lo = max(lo_last, read_lo);
     const int full_hi = hi_first;
-    auto compute = [&](int t, int b, auto full_tag) {
-      constexpr bool FULL = decltype(full_tag)::value;
+    // The pair of tiles t and t + 1; each operand's registers take the next pair's loads
+    // as soon as it is consumed.  Issues are unconditional -- past the last tile it is
+    // re-read (a cache hit) -- so no branch merges pending loads and the wait counts stay
+    // exact.
+    auto compute = [&](int t) {
       const int tb = w_begin + t * kTileTok;
-      const bool okv_k = FULL ? true : okk[b];
-      // ---- S^T = K Q^T : lane holds (positions tb + 4*grp + r, row l16 of tile nt)
-      f32x4 sc[NT];
+      const bool full = tb >= full_lo && tb + 2 * kTileTok <= full_hi;
+      // ---- S^T = K Q^T : lane holds (positions tb + 16 b + 4 * grp + r, row l16 of tile nt)
+      f32x4 sc[2][NT];
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) sc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int b = 0; b < 2; ++b) {
 #pragma unroll
-      for (int s = 0; s < NQS; ++s) {
-        const uint4 a = kb[b].op(s, okv_k);
+        for (int nt = 0; nt < NT; ++nt) sc[b][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) sc[nt] = M::qk(a, qreg[nt][s], sc[nt]);
+        for (int s = 0; s < NQS; ++s) {
+          const uint4 a = kb[b].op(s);
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) sc[b][nt] = M::mma(a, qreg[nt][s], sc[b][nt]);
+        }
       }
-      // positions past the sequence may hold any bits (NaN included): zero them
-      if (!FULL) {
+      issue_k(t + 2, 0);
+      if (!kLateKey) issue_k(t + 3, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      // ---- online softmax (log2 domain) and the P^T operand: contraction slots 8 grp + j
+      // hold positions 4 grp + j of tile t (j < 4) and 4 grp + j - 4 of tile t + 1
+      float vsc[2][4];
+      if (SM == 2) {
+        const float mine = inside(tb + (grp & 1) * kTileTok + l16) ? sraw : 0.f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (!(okv[b] >> i & 1u)) vq[b].zero(i);
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            vsc[b][r] = scale_of(mine, 2 + b, r);
+            const float ks = scale_of(mine, b, r);
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) sc[b][nt][r] *= ks;
+          }
       }
-      // ---- online softmax (log2 domain) and the P^T operand
-      uint2 pop[NT];
-      uint2 plo[CP ? NT : 1];
+      uint4 pop[NT];
+      uint4 plo[CP ? NT : 1];
       bool rescale = false;
       float corr[NT];
 #pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sc[b][nt][r] *= qk_scale;
+      if (!full) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int pos = tb + b * kTileTok + 4 * grp + r;
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+              sc[b][nt][r] = (pos >= row_lo[nt] && pos < row_hi[nt]) ? sc[b][nt][r] : -INFINITY;
+          }
+      }
+#pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
-        float sv4[4];
         float mx = -INFINITY;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          float x = sc[nt][r];
-          if (SM == 2) x *= ksc[b][r];
-          x *= qk_scale;
-          if (!FULL) {
-            const int pos = tb + 4 * grp + r;
-            x = (pos >= row_lo[nt] && pos < row_hi[nt]) ? x : -INFINITY;
-          }
-          sv4[r] = x;
-          mx = fmaxf(mx, x);
-        }
+        for (int r = 0; r < 8; ++r) mx = fmaxf(mx, sc[r >> 2][nt][r & 3]);
         mx = group_max(mx);
         const float m_new = fmaxf(m_run[nt], mx);
         // a row that has seen no visible key keeps m = -inf and weights 0
         const float m_use = m_new == -INFINITY ? 0.f : m_new;
         corr[nt] = m_new == m_run[nt] ? 1.f : __builtin_amdgcn_exp2f(m_run[nt] - m_use);
-        float pr[4];
+        float pr[8];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) pr[r] = __builtin_amdgcn_exp2f(sv4[r] - m_use);
+        for (int r = 0; r < 8; ++r) pr[r] = __builtin_amdgcn_exp2f(sc[r >> 2][nt][r & 3] - m_use);
         rescale |= corr[nt] != 1.f;
-        const float rs = group_sum(((pr[0] + pr[1]) + pr[2]) + pr[3]);
+        const float rs = group_sum(((pr[0] + pr[1]) + (pr[2] + pr[3])) +
+                                   ((pr[4] + pr[5]) + (pr[6] + pr[7])));
         l_run[nt] = l_run[nt] * corr[nt] + rs;
         m_run[nt] = m_new;
         if (SM == 2) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) pr[r] *= vsc[b][r];
+          for (int r = 0; r < 8; ++r) pr[r] *= vsc[r >> 2][r & 3];
         }
-        pop[nt].x = M::pack2(pr[0], pr[1]);
-        pop[nt].y = M::pack2(pr[2], pr[3]);
+        pop[nt] = make_uint4(M::pack2(pr[0], pr[1]), M::pack2(pr[2], pr[3]),
+                             M::pack2(pr[4], pr[5]), M::pack2(pr[6], pr[7]));
         if (CP) {
           // what the cast dropped, as a second 16-bit operand (the reference's
           // compensated dot, vllm_rlt/kernels/triton_attention.py:368-371)
-          plo[nt].x = M::pack2(pr[0] - M::lo_f32(pop[nt].x), pr[1] - M::hi_f32(pop[nt].x));
-          plo[nt].y = M::pack2(pr[2] - M::lo_f32(pop[nt].y), pr[3] - M::hi_f32(pop[nt].y));
+          auto dropped = [&](uint32_t w, int r) {
+            return M::pack2(pr[r] - M::lo_f32(w), pr[r + 1] - M::hi_f32(w));
+          };
+          plo[nt] = make_uint4(dropped(pop[nt].x, 0), dropped(pop[nt].y, 2),
+                               dropped(pop[nt].z, 4), dropped(pop[nt].w, 6));
         }
       }
+      issue_scales(t + 2);
+      __builtin_amdgcn_sched_barrier(0);
       // multiplying by exactly 1 changes no bit: skip the rescale when no row's
-      // running max moved in this tile (wave-uniform vote)
+      // running max moved in this pair (wave-uniform vote)
       if (__builtin_amdgcn_ballot_w64(rescale) != 0) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
           for (int dt = 0; dt < ND; ++dt) oacc[nt][dt] *= corr[nt];
       }
-      // ---- O^T += V^T P^T : A = V^T (dims ND * l16 + dt, positions 4grp..+3)
+      // positions outside the span may hold any bits (NaN included): zero them
+      if (!full) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (!inside(tb + b * kTileTok + 4 * grp + i)) vq[b].zero(i);
+      }
+      // ---- O^T += V^T P^T : A = V^T (dims ND * l16 + dt, positions as in P^T)
       for_pairs<ND, NT>([&](auto kc) {
         constexpr int K = decltype(kc)::value;
-        uint2 a0, a1;
-        vq[b].template op2<K>(a0, a1);
+        if (D > 128) __builtin_amdgcn_sched_barrier(0);  // (no registers left to run ahead)
+        uint2 a0, a1, b0, b1;
+        vq[0].template op2<K>(a0, a1);
+        vq[1].template op2<K>(b0, b1);
+        const uint4 v0 = make_uint4(a0.x, a0.y, b0.x, b0.y);
+        const uint4 v1 = make_uint4(a1.x, a1.y, b1.x, b1.y);
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-          oacc[nt][2 * K] = M::pv(a0, pop[nt], oacc[nt][2 * K]);
-          oacc[nt][2 * K + 1] = M::pv(a1, pop[nt], oacc[nt][2 * K + 1]);
+          oacc[nt][2 * K] = M::mma(v0, pop[nt], oacc[nt][2 * K]);
+          oacc[nt][2 * K + 1] = M::mma(v1, pop[nt], oacc[nt][2 * K + 1]);
           if (CP) {
-            oacc[nt][2 * K] = M::pv(a0, plo[nt], oacc[nt][2 * K]);
-            oacc[nt][2 * K + 1] = M::pv(a1, plo[nt], oacc[nt][2 * K + 1]);
+            oacc[nt][2 * K] = M::mma(v0, plo[nt], oacc[nt][2 * K]);
+            oacc[nt][2 * K + 1] = M::mma(v1, plo[nt], oacc[nt][2 * K + 1]);
           }
         }
       });
+      if (kLateKey) issue_k(t + 3, 1);
+      issue_v(t + 2, 0);
+      issue_v(t + 3, 1);
     };
-    auto step = [&](int t, int b) {
-      const int tb = w_begin + t * kTileTok;
-      const bool full = tb >= full_lo && tb + kTileTok <= full_hi;
-      if (full) compute(t, b, Flag<true>{});
-      else compute(t, b, Flag<false>{});
-    };
-    // kStages-deep pipeline: tile t + kStages is issued into the stage tile t just freed.
-    // Issues are unconditional -- past the last tile the last tile is re-read (a
-    // cache hit) -- so no branch merges pending loads and the wait counts stay exact.
-    const int tl = t1 - 1;
+    const int first = t0 & ~1;
 #pragma unroll
-    for (int b = 0; b < kStages; ++b) issue(min(t0 + b, tl), b);
-    for (int t = t0; t < t1; t += kStages) {
+    for (int b = 0; b < 2; ++b) issue_k(first + b, b);
+    issue_scales(first);
 #pragma unroll
-      for (int b = 0; b < kStages; ++b) {
-        if (b == 0 || t + b < t1) step(t + b, b);
-        issue(min(t + b + kStages, tl), b);
-      }
-    }
+    for (int b = 0; b < 2; ++b) issue_v(first + b, b);
+#pragma unroll 1
+    for (int t = first; t < t1; t += 2) compute(t);
   }
 
 }
@@ -1005,7 +1044,8 @@ __device__ __forceinline__ void unit_of(const AttnParams& P, const int32_t* firs
 // takes consecutive units instead -- neighbouring kv heads of one chunk -- so that the
 // lines two heads share reach the XCD's L2 once (16 windows of 5, 2048 positions, 55 heads
 // of 96 bf16 dims, 192 bytes each: every head fetched 2 lines for 1.5, and the launch ran
-// at the rate of those fetches, 6.4 TB/s; 151.6 -> 147.0 us).  kSlots units run at a time,
+// at the rate of those fetches, 6.4 TB/s; 151.6 -> 147.0 us).  So do the per-vector scales
+// of an fp8 pool, 4 bytes a head (64 windows at 8k, 8 heads: 278 -> 229 us).  kSlots units run at a time,
 // each on KS waves that split its positions and combine through LDS in a
 // fixed order, so a unit's arithmetic never depends on the assignment.
 template <int QT, int KVT, int D, int NT, int SM, bool UB, bool CP>
@@ -1580,14 +1620,19 @@ int launch_mfma_ub(const AttnParams& P, dim3 grid, int nt, hipStream_t stream) {
   return RLT_OK;
 }
 
-// Compensated P V is built for blocks holding whole 16-position tiles (the reference
-// pools' block size 16 and its multiples).
+// UB: blocks hold whole 16-position tiles and a lane's offset within a tile fits 32 bits.
+// Compensated P V is built for such block sizes only (the reference pools' block size 16
+// and its multiples).
 template <int QT, int KVT, int D, int SM>
 int launch_mfma_sm(const AttnParams& P, dim3 grid, int nt, hipStream_t stream) {
-  const bool ub = P.block_size % kTileTok == 0;
+  const bool whole = P.block_size % kTileTok == 0;
+  const int64_t most = (int64_t)1 << 26;
+  const bool ub = whole && P.k_token_stride >= 0 && P.k_token_stride < most &&
+                  P.v_token_stride >= 0 && P.v_token_stride < most;
   if (P.compensate) {
-    if (!ub) return RLT_ERR_UNSUPPORTED;
-    return launch_mfma_ub<QT, KVT, D, SM, true, true>(P, grid, nt, stream);
+    if (!whole) return RLT_ERR_UNSUPPORTED;
+    if (ub) return launch_mfma_ub<QT, KVT, D, SM, true, true>(P, grid, nt, stream);
+    return launch_mfma_ub<QT, KVT, D, SM, false, true>(P, grid, nt, stream);
   }
   if (ub) return launch_mfma_ub<QT, KVT, D, SM, true, false>(P, grid, nt, stream);
   return launch_mfma_ub<QT, KVT, D, SM, false, false>(P, grid, nt, stream);
@@ -1870,7 +1915,8 @@ int attention_impl(const void* q, int64_t q_row_stride, int64_t q_head_stride,
     const int64_t pairs = (int64_t)num_seqs * P.rowgroups;
     P.persistent = pairs <= kMaxPairs;
     P.shared_lines = num_kv_heads > 1 &&
-                     ((k_head_stride * kv_elt) % 128 != 0 || (v_head_stride * kv_elt) % 128 != 0);
+                     ((k_head_stride * kv_elt) % 128 != 0 || (v_head_stride * kv_elt) % 128 != 0 ||
+                      (scale_mode == 2 && s_head_stride * 4 < 128));
     int64_t wgs = (int64_t)num_seqs * P.rowgroups * num_kv_heads * P.max_chunks;
     if (P.persistent) wgs = compute_units();
     if (wgs >= ((int64_t)1 << 31)) return RLT_ERR_UNSUPPORTED;
