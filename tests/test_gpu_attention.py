@@ -1179,3 +1179,30 @@ def test_long_window_store_ragged_rows(kernel, pkg, dev, kv, d, hkv):
         assert torch.equal(got.view(torch.uint8), ref.view(torch.uint8))
     if kv == "fp8_vector":
         assert all(torch.equal(a, b) for a, b in zip(scales, want_scales))
+
+
+@pytest.mark.parametrize("kv,d", [("same", 96), ("fp8_vector", 64), ("fp8_vector", 128)])
+def test_full_rounds_of_neighbouring_heads_equal_single_rows(kernel, dev, kv, d):
+    """Batches that fill the persistent workgroups' rounds and whose heads share cache
+    lines (keys and values, or per-vector scales) take neighbouring heads together: every
+    row equals its own single-row call bit for bit."""
+    _say("neighbouring heads", kv, d)
+    g = torch.Generator(device=dev).manual_seed(d)
+    n, bs, hkv, width = 72, 16, 8, 256
+    shape = (n * width, bs, hkv, d)
+    if kv == "same":
+        k, v = (torch.randn(shape, generator=g, device=dev, dtype=torch.bfloat16)
+                for _ in range(2))
+        scales = ()
+    else:
+        k, v = (torch.randint(0, 120, shape, generator=g, device=dev, dtype=torch.uint8).view(
+            torch.float8_e4m3fn) for _ in range(2))
+        scales = tuple(torch.rand(shape[:-1], generator=g, device=dev) * 0.01 for _ in range(2))
+    tables = torch.randperm(n * width, generator=g, device=dev).int().view(n, width)
+    lengths = torch.randint(3500, 4097, (n,), generator=g, device=dev, dtype=torch.int32)
+    q = torch.randn(n, 2 * hkv, d, generator=g, device=dev, dtype=torch.bfloat16)
+    got = kernel(q, k, v, tables, lengths, *scales)
+    for i in (0, 35, n - 1):
+        one = kernel(q[i:i + 1], k, v, tables[i:i + 1], lengths[i:i + 1], *scales)
+        assert torch.equal(got[i:i + 1].view(torch.int16), one.view(torch.int16))
+    assert torch.isfinite(got).all()
