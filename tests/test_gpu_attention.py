@@ -1206,3 +1206,51 @@ def test_full_rounds_of_neighbouring_heads_equal_single_rows(kernel, dev, kv, d)
         one = kernel(q[i:i + 1], k, v, tables[i:i + 1], lengths[i:i + 1], *scales)
         assert torch.equal(got[i:i + 1].view(torch.int16), one.view(torch.int16))
     assert torch.isfinite(got).all()
+
+
+@pytest.mark.parametrize("dtype,half_ulp", [(torch.bfloat16, 2.0**-8), (torch.float16, 2.0**-11)])
+def test_weights_are_rounded_against_their_own_tiles_maximum(kernel, dev, dtype, half_ulp):
+    """A tile's largest weight is exactly 1 in the 16-bit operand, whatever follows: two
+    visible tokens, one in each of two neighbouring 16-position tiles, the second one's
+    score higher by delta, values 1 and 0.  The output is c / (1 + c), c = e^-delta, formed
+    in fp32 and rounded once: half an ulp of the 16-bit type (2^-8 or 2^-11 of the value's
+    power of two), and 2^-20 for the fp32 steps.  A maximum shared by both tiles would round
+    c as well."""
+    _say("own maximum", dtype)
+    d, bs, n = 64, 16, 64
+    k = torch.full((2 * n, bs, 1, d), 0.0, dtype=dtype)
+    v = torch.zeros(2 * n, bs, 1, d, dtype=dtype)
+    k[..., 0] = -64.0                       # e^-64: no share in the output
+    delta = torch.arange(1, n + 1) / 32.0   # exact in both types
+    k[0::2, 3, 0, 0] = 0.0
+    v[0::2, 3] = 1.0
+    k[1::2, 5, 0, 0] = delta.to(dtype)
+    q = torch.zeros(n, 1, d, dtype=dtype)
+    q[..., 0] = d ** 0.5                    # score = key
+    tables = torch.arange(2 * n, dtype=torch.int32).view(n, 2)
+    lengths = torch.full((n,), 2 * bs, dtype=torch.int32)
+    got = kernel(q.to(dev), k.to(dev), v.to(dev), tables.to(dev), lengths.to(dev)).cpu().double()
+    c = (-delta.double()).exp()
+    want = (c / (1 + c)).view(n, 1, 1).expand(n, 1, d)
+    bound = half_ulp * 2.0 ** want.log2().floor() + want * 2.0**-20
+    assert ((got - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("bs", [8, 16, 48])
+@pytest.mark.parametrize("d", [64, 256])
+def test_sliding_windows_from_every_tile_of_a_span(kernel, dev, bs, d):
+    """Windows whose first tile is an odd or even one of its span and whose last tile ends
+    the span, the chunk or the sequence (tiles go in pairs, and a pair's second tile may lie
+    past the span), against the oracle."""
+    _say("window tiles", bs, d)
+    g = torch.Generator().manual_seed(bs + d)
+    hkv, hq, lengths = 2, 4, [255, 256, 257, 272, 511, 512, 513, 530, 768, 1024, 1030]
+    pages = sum(-(-n // bs) for n in lengths)
+    kpool, vpool, k, v = make_pool(pages, 2, bs, hkv, d, torch.bfloat16, g, layer=1)
+    tables = random_tables(lengths, bs, pages, g)
+    ctx = torch.tensor(lengths, dtype=torch.int32)
+    q = torch.randn(len(lengths), hq, d, generator=g).bfloat16()
+    for window in (1, 16, 17, 40, 250, 258, 300):
+        got = kernel.windowed(q.to(dev), kpool.to(dev)[:, 1], vpool.to(dev)[:, 1], tables.to(dev),
+                              ctx.to(dev), window)
+        _close(got, oatt.paged_attention(q, k, v, tables, ctx, window=window), torch.bfloat16)

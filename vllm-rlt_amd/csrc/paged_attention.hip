@@ -35,14 +35,18 @@
 //    S^T = K Q^T with v_mfma_f32_16x16x32_{bf16,f16} straight from global memory
 //    (the contraction order is permuted so that each lane's eight elements per
 //    step are contiguous in memory: the A-operand layout), online softmax in fp32
-//    (log2 domain), then O^T = V^T P^T with the same instruction over a pair of
-//    tiles: the P^T operand is the pair's S^T accumulators as they lie (the contraction
-//    order is free), and the output dimensions are permuted so that V^T operands are
-//    contiguous loads too (no LDS transpose).  A pair at a time because the step is a
-//    serial chain -- scores, maximum over lanes, exponentials, sum over lanes, products --
-//    that a wave alone on its SIMD waits through (0.48 us per 16 positions before).  One
-//    row at 700 positions, 16 heads: 17.4 -> 15.6 us; 8 rows of fp8 at 2-4k: 49 -> 38;
-//    windows of 5 at up to 8k: 80.8 -> 79.0; 64 x 4 planes of fp8 at 16-32k: 2.51 -> 2.43 ms.
+//    (log2 domain), then O^T = V^T P^T with v_mfma_f32_16x16x16: the P^T operand is the
+//    S^T accumulator as it lies (the contraction order is free), and the output dimensions
+//    are permuted so that V^T operands are contiguous loads too (no LDS transpose).  Tiles
+//    go in pairs because the step is a serial chain -- scores, maximum over lanes,
+//    exponentials, sum over lanes, products -- that a wave alone on its SIMD waits through
+//    (0.48 us per 16 positions one at a time): the pair's scores, lane reductions and
+//    exponentials run side by side.  The second tile's maximum, sums and products still
+//    follow the first's: one maximum for both would round the weight of every tile's
+//    largest token that is not the pair's (it is exactly 1 against its own), which put the
+//    output 0.4% further off float64.  One row at 700 positions, 16 heads: 17.8 -> 16.6 us;
+//    8 windows of 5 over fp8 at 2-4k: 57 -> 49.6; 64 x 4 planes of fp8 at 16-32k: 2.43 ->
+//    2.38 ms.  (With one maximum a pair: 16.1, 49.0, 2.37.)
 //  * vector (fp32 q, or any other head_dim <= 256): fp32 FMA dot products.
 
 #include "common.h"
@@ -225,6 +229,7 @@ __device__ __forceinline__ void merge_scales(float m1, float m2, float& mo, floa
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 template <int QT>
@@ -232,11 +237,17 @@ struct Mfma;
 
 template <>
 struct Mfma<RLT_BF16> {
-  __device__ static f32x4 mma(uint4 a, uint4 b, f32x4 c) {
+  __device__ static f32x4 qk(uint4 a, uint4 b, f32x4 c) {
     bf16x8 av, bv;
     __builtin_memcpy(&av, &a, 16);
     __builtin_memcpy(&bv, &b, 16);
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, c, 0, 0, 0);
+  }
+  __device__ static f32x4 pv(uint2 a, uint2 b, f32x4 c) {
+    s16x4 av, bv;
+    __builtin_memcpy(&av, &a, 8);
+    __builtin_memcpy(&bv, &b, 8);
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, c, 0, 0, 0);
   }
   __device__ static uint16_t from_f32(float x) { return f32_to_bf16_bits(x); }
   // the two values of a packed pair, exactly
@@ -252,11 +263,17 @@ struct Mfma<RLT_BF16> {
 
 template <>
 struct Mfma<RLT_F16> {
-  __device__ static f32x4 mma(uint4 a, uint4 b, f32x4 c) {
+  __device__ static f32x4 qk(uint4 a, uint4 b, f32x4 c) {
     f16x8 av, bv;
     __builtin_memcpy(&av, &a, 16);
     __builtin_memcpy(&bv, &b, 16);
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bv, c, 0, 0, 0);
+  }
+  __device__ static f32x4 pv(uint2 a, uint2 b, f32x4 c) {
+    f16x4 av, bv;
+    __builtin_memcpy(&av, &a, 8);
+    __builtin_memcpy(&bv, &b, 8);
+    return __builtin_amdgcn_mfma_f32_16x16x16f16(av, bv, c, 0, 0, 0);
   }
   __device__ static uint16_t from_f32(float x) { return f32_to_f16_bits(x); }
   __device__ static float lo_f32(uint32_t w) { return f16_bits_to_f32((uint16_t)(w & 0xffffu)); }
@@ -682,14 +699,13 @@ __device__ __forceinline__ void attend_span(const AttnParams& P, int seq, int rg
     const int64_t k_head = (int64_t)kvh * P.k_head_stride + grp * Raw::kGroupElems;
     const int64_t v_head = (int64_t)kvh * P.v_head_stride + l16 * ND;
     const int32_t* tbl = tbl_lds - c_begin;  // tbl[pos] for pos in the chunk
-    // positions of the span's tiles: [read_lo, hi_last); the others of a pair are masked,
-    // their values taken as zeros (they may hold any bits, NaN included)
-    const int read_lo = w_begin + t0 * kTileTok;
-    auto inside = [&](int pos) { return pos >= read_lo && pos < hi_last; };
-    // Loads of tile t into half b of the pair.  Branch-free: the tile is clamped into the
-    // span's tiles, so every address is one that some row reads.
+    // positions from hi_last on are masked, their values taken as zeros (they may hold any
+    // bits, NaN included)
+    auto inside = [&](int pos) { return pos < hi_last; };
+    // Loads of tile t into half b of the pair.  Branch-free: past the span's last tile it
+    // is that tile's, so every address is one that some row reads.
     const int tl = t1 - 1;
-    auto tile_base = [&](int t) { return w_begin + min(max(t, t0), tl) * kTileTok; };
+    auto tile_base = [&](int t) { return w_begin + min(t, tl) * kTileTok; };
     // With whole tiles per block the block is wave-uniform: a scalar base and a 32-bit lane
     // offset (fewer address registers; launch_mfma_sm bounds the strides).
     const uint32_t k_lane = (uint32_t)(l16 * (uint32_t)P.k_token_stride + grp * Raw::kGroupElems) * KV_ELT;
@@ -749,12 +765,16 @@ __device__ __forceinline__ void attend_span(const AttnParams& P, int seq, int rg
     // first row) is visible to every row of the row-group and fully stored, so
     // it needs no position masks.  (Branches around the masks: two copies of the whole
     // step, one without them, cost registers that D = 256 and two row tiles do not have.)
-    const int full_lo = max(lo_last, read_lo);
-    const int full_hi = hi_first;
+    // A pair whose second tile lies past the span's is never full, and that tile is masked.
+    const int span_end = w_begin + kSpan;
+    const int full_lo = lo_last;
+    const int full_hi = min(hi_first, span_end);
     // The pair of tiles t and t + 1; each operand's registers take the next pair's loads
     // as soon as it is consumed.  Issues are unconditional -- past the last tile it is
     // re-read (a cache hit) -- so no branch merges pending loads and the wait counts stay
-    // exact.
+    // exact.  The two tiles share the step's latencies, not its arithmetic: the running
+    // maximum, the sums and the products of tile t + 1 follow those of tile t, so a row's
+    // bits do not depend on where its pairs begin.
     auto compute = [&](int t) {
       const int tb = w_begin + t * kTileTok;
       const bool full = tb >= full_lo && tb + 2 * kTileTok <= full_hi;
@@ -768,14 +788,14 @@ __device__ __forceinline__ void attend_span(const AttnParams& P, int seq, int rg
         for (int s = 0; s < NQS; ++s) {
           const uint4 a = kb[b].op(s);
 #pragma unroll
-          for (int nt = 0; nt < NT; ++nt) sc[b][nt] = M::mma(a, qreg[nt][s], sc[b][nt]);
+          for (int nt = 0; nt < NT; ++nt) sc[b][nt] = M::qk(a, qreg[nt][s], sc[b][nt]);
         }
       }
       issue_k(t + 2, 0);
       if (!kLateKey) issue_k(t + 3, 1);
       __builtin_amdgcn_sched_barrier(0);
-      // ---- online softmax (log2 domain) and the P^T operand: contraction slots 8 grp + j
-      // hold positions 4 grp + j of tile t (j < 4) and 4 grp + j - 4 of tile t + 1
+      // ---- online softmax (log2 domain) and the P^T operands: contraction slot 4 grp + j
+      // of tile b holds its position 4 grp + j
       float vsc[2][4];
       if (SM == 2) {
         const float mine = inside(tb + (grp & 1) * kTileTok + l16) ? sraw : 0.f;
@@ -789,10 +809,10 @@ __device__ __forceinline__ void attend_span(const AttnParams& P, int seq, int rg
             for (int nt = 0; nt < NT; ++nt) sc[b][nt][r] *= ks;
           }
       }
-      uint4 pop[NT];
-      uint4 plo[CP ? NT : 1];
-      bool rescale = false;
-      float corr[NT];
+      uint2 pop[2][NT];
+      uint2 plo[2][CP ? NT : 1];
+      bool rescale[2] = {false, false};
+      float corr[2][NT];
 #pragma unroll
       for (int b = 0; b < 2; ++b)
 #pragma unroll
@@ -807,53 +827,50 @@ __device__ __forceinline__ void attend_span(const AttnParams& P, int seq, int rg
             const int pos = tb + b * kTileTok + 4 * grp + r;
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
-              sc[b][nt][r] = (pos >= row_lo[nt] && pos < row_hi[nt]) ? sc[b][nt][r] : -INFINITY;
+              sc[b][nt][r] = (pos >= row_lo[nt] && pos < min(row_hi[nt], span_end)) ? sc[b][nt][r] : -INFINITY;
           }
       }
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
-        float mx = -INFINITY;
+        float mx[2], rs[2], pr[2][4];
 #pragma unroll
-        for (int r = 0; r < 8; ++r) mx = fmaxf(mx, sc[r >> 2][nt][r & 3]);
-        mx = group_max(mx);
-        const float m_new = fmaxf(m_run[nt], mx);
-        // a row that has seen no visible key keeps m = -inf and weights 0
-        const float m_use = m_new == -INFINITY ? 0.f : m_new;
-        corr[nt] = m_new == m_run[nt] ? 1.f : __builtin_amdgcn_exp2f(m_run[nt] - m_use);
-        float pr[8];
-#pragma unroll
-        for (int r = 0; r < 8; ++r) pr[r] = __builtin_amdgcn_exp2f(sc[r >> 2][nt][r & 3] - m_use);
-        rescale |= corr[nt] != 1.f;
-        const float rs = group_sum(((pr[0] + pr[1]) + (pr[2] + pr[3])) +
-                                   ((pr[4] + pr[5]) + (pr[6] + pr[7])));
-        l_run[nt] = l_run[nt] * corr[nt] + rs;
-        m_run[nt] = m_new;
-        if (SM == 2) {
-#pragma unroll
-          for (int r = 0; r < 8; ++r) pr[r] *= vsc[r >> 2][r & 3];
+        for (int b = 0; b < 2; ++b) {
+          mx[b] = fmaxf(fmaxf(sc[b][nt][0], sc[b][nt][1]), fmaxf(sc[b][nt][2], sc[b][nt][3]));
+          mx[b] = group_max(mx[b]);
         }
-        pop[nt] = make_uint4(M::pack2(pr[0], pr[1]), M::pack2(pr[2], pr[3]),
-                             M::pack2(pr[4], pr[5]), M::pack2(pr[6], pr[7]));
-        if (CP) {
-          // what the cast dropped, as a second 16-bit operand (the reference's
-          // compensated dot, vllm_rlt/kernels/triton_attention.py:368-371)
-          auto dropped = [&](uint32_t w, int r) {
-            return M::pack2(pr[r] - M::lo_f32(w), pr[r + 1] - M::hi_f32(w));
-          };
-          plo[nt] = make_uint4(dropped(pop[nt].x, 0), dropped(pop[nt].y, 2),
-                               dropped(pop[nt].z, 4), dropped(pop[nt].w, 6));
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          const float m_new = fmaxf(m_run[nt], mx[b]);
+          // a row that has seen no visible key keeps m = -inf and weights 0
+          const float m_use = m_new == -INFINITY ? 0.f : m_new;
+          corr[b][nt] = m_new == m_run[nt] ? 1.f : __builtin_amdgcn_exp2f(m_run[nt] - m_use);
+          rescale[b] |= corr[b][nt] != 1.f;
+          m_run[nt] = m_new;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) pr[b][r] = __builtin_amdgcn_exp2f(sc[b][nt][r] - m_use);
+        }
+#pragma unroll
+        for (int b = 0; b < 2; ++b) rs[b] = group_sum(((pr[b][0] + pr[b][1]) + pr[b][2]) + pr[b][3]);
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          l_run[nt] = l_run[nt] * corr[b][nt] + rs[b];
+          if (SM == 2) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) pr[b][r] *= vsc[b][r];
+          }
+          pop[b][nt] = make_uint2(M::pack2(pr[b][0], pr[b][1]), M::pack2(pr[b][2], pr[b][3]));
+          if (CP) {
+            // what the cast dropped, as a second 16-bit operand (the reference's
+            // compensated dot, vllm_rlt/kernels/triton_attention.py:368-371)
+            auto dropped = [&](uint32_t w, int r) {
+              return M::pack2(pr[b][r] - M::lo_f32(w), pr[b][r + 1] - M::hi_f32(w));
+            };
+            plo[b][nt] = make_uint2(dropped(pop[b][nt].x, 0), dropped(pop[b][nt].y, 2));
+          }
         }
       }
       issue_scales(t + 2);
       __builtin_amdgcn_sched_barrier(0);
-      // multiplying by exactly 1 changes no bit: skip the rescale when no row's
-      // running max moved in this pair (wave-uniform vote)
-      if (__builtin_amdgcn_ballot_w64(rescale) != 0) {
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-          for (int dt = 0; dt < ND; ++dt) oacc[nt][dt] *= corr[nt];
-      }
       // positions outside the span may hold any bits (NaN included): zero them
       if (!full) {
 #pragma unroll
@@ -862,37 +879,48 @@ __device__ __forceinline__ void attend_span(const AttnParams& P, int seq, int rg
           for (int i = 0; i < 4; ++i)
             if (!inside(tb + b * kTileTok + 4 * grp + i)) vq[b].zero(i);
       }
-      // ---- O^T += V^T P^T : A = V^T (dims ND * l16 + dt, positions as in P^T)
-      for_pairs<ND, NT>([&](auto kc) {
-        constexpr int K = decltype(kc)::value;
-        if (D > 128) __builtin_amdgcn_sched_barrier(0);  // (no registers left to run ahead)
-        uint2 a0, a1, b0, b1;
-        vq[0].template op2<K>(a0, a1);
-        vq[1].template op2<K>(b0, b1);
-        const uint4 v0 = make_uint4(a0.x, a0.y, b0.x, b0.y);
-        const uint4 v1 = make_uint4(a1.x, a1.y, b1.x, b1.y);
+      // ---- O^T += V^T P^T, tile by tile : A = V^T (dims ND * l16 + dt, positions as in P^T)
+      auto product = [&](auto bc) {
+        constexpr int B = decltype(bc)::value;
+        // multiplying by exactly 1 changes no bit: skip the rescale when no row's
+        // running max moved in this tile (wave-uniform vote)
+        if (__builtin_amdgcn_ballot_w64(rescale[B]) != 0) {
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-          oacc[nt][2 * K] = M::mma(v0, pop[nt], oacc[nt][2 * K]);
-          oacc[nt][2 * K + 1] = M::mma(v1, pop[nt], oacc[nt][2 * K + 1]);
-          if (CP) {
-            oacc[nt][2 * K] = M::mma(v0, plo[nt], oacc[nt][2 * K]);
-            oacc[nt][2 * K + 1] = M::mma(v1, plo[nt], oacc[nt][2 * K + 1]);
-          }
+          for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int dt = 0; dt < ND; ++dt) oacc[nt][dt] *= corr[B][nt];
         }
-      });
-      if (kLateKey) issue_k(t + 3, 1);
+        for_pairs<ND, NT>([&](auto kc) {
+          constexpr int K = decltype(kc)::value;
+          if (D > 128) __builtin_amdgcn_sched_barrier(0);  // (no registers left to run ahead)
+          uint2 a0, a1;
+          vq[B].template op2<K>(a0, a1);
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) {
+            oacc[nt][2 * K] = M::pv(a0, pop[B][nt], oacc[nt][2 * K]);
+            oacc[nt][2 * K + 1] = M::pv(a1, pop[B][nt], oacc[nt][2 * K + 1]);
+            if (CP) {
+              oacc[nt][2 * K] = M::pv(a0, plo[B][nt], oacc[nt][2 * K]);
+              oacc[nt][2 * K + 1] = M::pv(a1, plo[B][nt], oacc[nt][2 * K + 1]);
+            }
+          }
+        });
+      };
+      product(std::integral_constant<int, 0>{});
+      if (t + 1 < t1) product(std::integral_constant<int, 1>{});  // (wave-uniform)
+      if (kLateKey) {
+        issue_k(t + 3, 1);
+      }
       issue_v(t + 2, 0);
       issue_v(t + 3, 1);
     };
-    const int first = t0 & ~1;
 #pragma unroll
-    for (int b = 0; b < 2; ++b) issue_k(first + b, b);
-    issue_scales(first);
+    for (int b = 0; b < 2; ++b) issue_k(t0 + b, b);
+    issue_scales(t0);
 #pragma unroll
-    for (int b = 0; b < 2; ++b) issue_v(first + b, b);
+    for (int b = 0; b < 2; ++b) issue_v(t0 + b, b);
 #pragma unroll 1
-    for (int t = first; t < t1; t += 2) compute(t);
+    for (int t = t0; t < t1; t += 2) compute(t);
   }
 
 }
