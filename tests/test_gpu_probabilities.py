@@ -779,3 +779,43 @@ def test_filter_form_in_verify_and_draft_calls(pkg, dev, vocab, dtype, flat):
     expected = logits.float().argmax(-1)
     expected[some[:4]] = drawn
     assert torch.equal(proposed, expected)
+
+
+@pytest.mark.parametrize("kind", ["k", "p", "kp"])
+@pytest.mark.parametrize("temp,tops,tie", [(0.84501016, (18.75, 14.625), 11.6875),
+                                           (0.86269689, (43.0, 42.5), 38.25),
+                                           (1.65, (17.125, 16.0), 7.40625)])
+def test_filter_form_equal_logits_in_slices_of_different_maxima(pkg, dev, kind, temp, tops, tie):
+    """Equal logits in two slices of a split row, whose slices' maxima differ: the cut takes
+    them in column order, as everywhere.  At these temperatures and logits their masses
+    relative to the two slices' rounded maxima lie on two sides of a histogram bin's edge.
+    The kept tokens are counted (3 and 4, the tie's first column alone and both), and the
+    row sums to 1 (2^-20: fp32 values of at most four tokens)."""
+    _say("filter form ties", kind, temp)
+    vocab = 81928
+    k_of, p_of, rows, kept = [], [], [], []
+    for first, second in ((0, 1), (1, 0)):
+        x = torch.full((vocab,), -30.0)
+        x[100], x[9000] = tops[first], tops[second]
+        x[5], x[8200] = tie, tie
+        e = ((x.double() - x.max().double()) / temp).exp()
+        total = float(e.sum())
+        # half of a tie's mass past the first k tokens
+        mass = [float(e[100] + e[9000] + (i - 0.5) * e[5]) / total for i in range(3)]
+        for n in (3, 4):
+            rows.append(x)
+            k_of.append(n if "k" in kind else -1)
+            p_of.append(mass[n - 2] if "p" in kind else 1.0)
+            kept.append([100, 9000, 5, 8200][:n])
+    if kind == "kp":
+        # the top-k cut after the tie, the top-p cut inside it (mass over the k survivors)
+        k_of = [4] * len(rows)
+    logits = torch.stack(rows).to(dev)
+    t = torch.full((len(rows),), temp)
+    k = torch.tensor(k_of)
+    p = torch.tensor(p_of)
+    plan = _host_args(k.tolist(), p.tolist(), vocab)
+    got = pkg.batched_probabilities(logits, t.to(dev), k.to(dev), p.to(dev), **plan).cpu()
+    for r, want in enumerate(kept):
+        assert sorted(got[r].nonzero().view(-1).tolist()) == sorted(want), f"row {r}"
+        assert abs(float(got[r].double().sum()) - 1) <= 2.0**-20, f"row {r}"

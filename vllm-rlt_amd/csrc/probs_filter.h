@@ -26,14 +26,22 @@
 //
 // Masses.  With c = log2(e) / T and A_s the slice's anchor (its maximum's l c, rounded to an
 // integer), a token's mass is e = 2^(l c - A_s) (one fma, then the hardware exponential); the
-// largest lies in [0.7, 1.42).  Anchors are integers, so a row's masses are its slices' times
-// powers of two.  Octave o of e is [2^-o, 2^(1-o)); a histogram has 64 bins in each of octaves
-// 0 .. 24 and 4 in each of 25 .. 126, and a slice whose anchor is d below the row's moves d
-// octaves on.  A bin's masses are 24-bit integers times one power of two and at most 2^18 of
-// them, so float64 sums of a bin (or an octave) are exact in any order.
+// largest lies in [0.69, 1.45).  Anchors are integers, so a row's masses are its slices' times
+// powers of two.
+//
+// Bins.  A token's bin comes from floor(64 l c), the product rounded once to fp32: it never
+// falls as l grows, and equal logits share it in every slice, so bins agree with the order in
+// which tokens are kept and written.  (Bins taken from the masses did not: the fma rounds
+// l c - A_s by the slice's anchor, equal logits of two slices could fall on two sides of a
+// bin's edge, and a row then kept one token more or less than it counted.)  Octave o of a
+// slice holds the tokens with l c - A_s in [-o, 1 - o), a histogram has 64 bins in each of
+// octaves 0 .. 24 and 4 in each of 25 .. 125, and a slice whose anchor is d below the row's
+// moves d octaves on.  l c is rounded by at most 2^-5 (|l c| <= 2^20), so a bin's masses are
+// within 7% of each other: 25-bit integers times one power of two, at most 2^18 of them, whose
+// float64 sums are exact in any order (so are an octave's).
 //
 // Depth.  A slice's histogram ends at octave 16 unless a cut may lie deeper: at 24 when the
-// mass below octave 16 exceeds half of the 1 - p that a top-p cut may drop, at 126 when the
+// mass below octave 16 exceeds half of the 1 - p that a top-p cut may drop, at 125 when the
 // slice has fewer than k tokens in octaves 0 .. 16 (with k of them, the row's k-th token lies
 // there too).  Rows that this form does not decide -- a cut below a slice's histogram, more
 // tokens in the cut bins than the list holds (flat rows, large tie groups), logits out of
@@ -51,7 +59,7 @@ constexpr int kWaves = kThreads / RLT_WAVE;
 constexpr int E = 32;                // columns per thread
 constexpr int kSlice = kThreads * E; // 8192: also one group of the cascade row sums
 constexpr int kMaxSlices = 32;
-constexpr int kOctaves = 127;        // [0, 127): normal floats below 2
+constexpr int kOctaves = 126;        // [0, 126): their masses are normal floats
 constexpr int kFine = 25;            // octaves of 64 bins; the others have 4
 constexpr int kShallow = 16;         // last octave of the usual histogram
 constexpr int kFineBins = 64, kCoarseBins = 4;
@@ -143,18 +151,21 @@ __device__ __forceinline__ float mass_of(float l, float c, float anchor) {
   return __builtin_amdgcn_exp2f(__builtin_fmaf(l, c, -anchor));
 }
 
-// Smallest float bits of octave o.
-__device__ __forceinline__ uint32_t octave_floor(int o) { return 0x3f800000u - ((uint32_t)o << 23); }
 // First bin of octave o.
 __device__ __forceinline__ int octave_bin(int o) {
   return o < kFine ? o * kFineBins : kFine * kFineBins + (o - kFine) * kCoarseBins;
 }
-// Bin of a mass from its bits (below 2): larger masses first.  Masses below octave 126 lie
-// past every bin.
-__device__ __forceinline__ int bin_of_bits(uint32_t bits) {
-  const uint32_t d = 0x3fffffffu - bits;
-  const int fine = (int)(d >> 17);
-  return fine < kFine * kFineBins ? fine : kFine * kFineBins + (int)((d >> 21) - kFine * kCoarseBins);
+// Step of logit l below `anchor`: 64 to the octave, 0 the first of octave 0 (a slice's own
+// logits start at 31).  -inf, which pads the row, and logits far below lie past every octave.
+__device__ __forceinline__ int step_of(float l, float c, int anchor) {
+  return 64 * (anchor + 1) - 1 - (int)floorf(64.f * fmaxf(l * c, -4.f * kMaxScaled));
+}
+// Bin of a step, and the first step of a bin.
+__device__ __forceinline__ int bin_of_step(int f) {
+  return f < kFine * kFineBins ? f : kFine * kFineBins + ((f - kFine * kFineBins) >> 4);
+}
+__device__ __forceinline__ int first_step(int b) {
+  return b < kFine * kFineBins ? b : kFine * kFineBins + ((b - kFine * kFineBins) << 4);
 }
 
 // Element j of thread t in a slice at column c0: c0 + 4 (256 (j / 4) + t) + j % 4.
@@ -354,29 +365,34 @@ __global__ __launch_bounds__(kThreads, 4) void rlt_filter_slice_kernel(
     }
     return;
   }
-  // masses in place of the logits, their total, and the histogram of octaves 0 .. kShallow
+  // the masses' total and the histogram of octaves 0 .. kShallow
   const float fa = (float)anchor;
   const bool cuts = rule.do_k || rule.do_p;
   double z = 0.0;
-#pragma unroll
-  for (int j = 0; j < E; ++j) {
-    x[j] = mass_of(x[j], rule.c, fa);
-    z += (double)x[j];
-  }
-  // (one pass with counts, one without: a branch on it per token cost as much as the rest)
-  auto add = [&](uint32_t lo, uint32_t hi, auto counts) {  // masses with bits in [lo, hi)
+  // tokens with steps in [lo, hi) go to the histogram (one pass with counts, one without: a
+  // branch on it per token cost as much as the rest)
+  auto add = [&](int lo, int hi, auto counts, auto total) {
 #pragma unroll
     for (int j = 0; j < E; ++j) {
-      const uint32_t bits = __float_as_uint(x[j]);
-      if (bits - lo < hi - lo) {
-        const int b = (int)((0x3fffffffu - bits) >> 17);  // a fine one
-        atomicAdd(&sh.mass[b], (double)x[j]);
+      const float e = mass_of(x[j], rule.c, fa);
+      if constexpr (decltype(total)::value) z += (double)e;
+      const int f = step_of(x[j], rule.c, anchor);
+      if ((uint32_t)(f - lo) < (uint32_t)(hi - lo)) {
+        const int b = bin_of_step(f);
+        atomicAdd(&sh.mass[b], (double)e);
         if constexpr (decltype(counts)::value) atomicAdd(&sh.cnt[b], 1u);
       }
     }
   };
-  if (rule.do_k) add(octave_floor(kShallow), 0x40000000u, std::true_type{});
-  else if (rule.do_p) add(octave_floor(kShallow), 0x40000000u, std::false_type{});
+  constexpr int kShallowSteps = (kShallow + 1) * kFineBins;
+  if (rule.do_k) {
+    add(0, kShallowSteps, std::true_type{}, std::true_type{});
+  } else if (rule.do_p) {
+    add(0, kShallowSteps, std::false_type{}, std::true_type{});
+  } else {
+#pragma unroll
+    for (int j = 0; j < E; ++j) z += (double)mass_of(x[j], rule.c, fa);
+  }
   z = lane_sum(z);
   if (lane == 0) sh.z[w] = z;
   __syncthreads();
@@ -423,16 +439,7 @@ __global__ __launch_bounds__(kThreads, 4) void rlt_filter_slice_kernel(
     if (rule.do_p && z - top > 0.5 * (1.0 - (double)rule.p) * z) depth = kFine - 1;
     if (rule.do_k && n_top < rule.kk) depth = kOctaves - 1;
     if (depth > kShallow) {  // uniform over the workgroup
-      const uint32_t lo = octave_floor(depth), hi = octave_floor(kShallow);
-#pragma unroll
-      for (int j = 0; j < E; ++j) {
-        const uint32_t bits = __float_as_uint(x[j]);
-        if (bits >= lo && bits < hi) {
-          const int b = bin_of_bits(bits);
-          atomicAdd(&sh.mass[b], (double)x[j]);
-          atomicAdd(&sh.cnt[b], 1u);
-        }
-      }
+      add(kShallowSteps, (depth + 1) * kFineBins, std::true_type{}, std::false_type{});
       __syncthreads();
 #pragma unroll 1
       for (int o = kShallow + 1 + w; o < kFine; o += kWaves) put(o);
@@ -696,13 +703,11 @@ __device__ __forceinline__ RowCut row_cut(const View& v, const Rule& rule, int64
     cut.mass_before = lo.mass_before;
   }
   cut.state = kCut;
-  // the logits of bins b_lo .. max(b_hi, k_bin), widened by more than what the masses'
-  // fma and exponential and this inverse may be off (in log2 units)
+  // the logits of bins b_lo .. max(b_hi, k_bin), widened by more than what the product and
+  // this quotient round
   const float slack = 1e-3f + 1e-6f * fabsf((float)anchor);
-  auto edge = [&](int bin) {  // upper edge of a bin's masses, log2
-    const uint32_t d = bin < kFine * kFineBins ? (uint32_t)bin << 17
-                                               : (uint32_t)(bin - kFine * (kFineBins - kCoarseBins)) << 21;
-    return __builtin_amdgcn_logf(__uint_as_float(0x3fffffffu - min(d, 0x3f7fffffu))) + (float)anchor;
+  auto edge = [&](int bin) {  // upper edge of a bin's l c
+    return (float)(anchor + 1) - (float)first_step(bin) * (1.f / kFineBins);
   };
   cut.l_hi = (edge(cut.b_lo) + slack) / rule.c;
   cut.l_lo = (edge(max(cut.b_hi, cut.k_bin) + 1) - slack) / rule.c;
@@ -717,6 +722,11 @@ __device__ __forceinline__ double block_sum(RowShared& sh, double x) {
   for (int i = 0; i < kRowWaves; ++i) x += sh.sum[i];
   __syncthreads();
   return x;
+}
+
+// Bin of a listed token, from its logit.
+__device__ __forceinline__ int listed_bin(unsigned long long at, const Rule& rule, const RowCut& cut) {
+  return bin_of_step(step_of(key_value(~(uint32_t)(at >> 32)), rule.c, cut.anchor));
 }
 
 // Decides the n listed tokens (in no particular order: ranks and masses before a token are
@@ -742,7 +752,7 @@ __device__ __forceinline__ double pick_listed(RowShared& sh, const RowCut& cut, 
     double others = 0.0;
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
-      in_k[i] = keep[i] && bin_of_bits(__float_as_uint((float)own[i].mass)) == cut.k_bin;
+      in_k[i] = keep[i] && listed_bin(own[i].at, rule, cut) == cut.k_bin;
       others += keep[i] && !in_k[i] ? 1.0 : 0.0;
       rank[i] = 0;
     }
@@ -823,7 +833,7 @@ __device__ __forceinline__ void pick_few(RowShared& sh, const RowCut& cut, const
     return ((unsigned long long)hi << 32) | lo;
   };
   if (rule.do_k) {
-    const bool in_k = keep && bin_of_bits(__float_as_uint((float)own.mass)) == cut.k_bin;
+    const bool in_k = keep && listed_bin(own.at, rule, cut) == cut.k_bin;
     uint32_t rank = 0;
     for (int j = 0; j < n; ++j) rank += other(own.at, j) < own.at;
     const uint32_t before = (uint32_t)__popcll(__ballot(keep && !in_k));
@@ -902,18 +912,17 @@ __global__ __launch_bounds__(kRowThreads) void rlt_filter_row_kernel(
   if (t == 0) sh.list_n = 0;
   __syncthreads();
   if (cut.state == kCut) {
-    // the tokens of the cut bins: a look at the logit first, then the bin by the mass of the
-    // token's own slice, as its histogram counted it
+    // the tokens of the cut bins (a look at the logit first), each with the mass that its own
+    // slice's histogram counted
     auto look = [&](float l, uint32_t col) {
       if (!(l >= cut.l_lo && l <= cut.l_hi)) return;
-      const int a = sh.anchor[col / kSlice];
-      const uint32_t bits = __float_as_uint(mass_of(l, rule.c, (float)a));
-      const uint32_t shift = (uint32_t)min(cut.anchor - a, 255) << 23;
-      const int b = bits >= shift ? bin_of_bits(bits - shift) : kBins;
+      const int b = bin_of_step(step_of(l, rule.c, cut.anchor));
       if (!((b >= cut.b_lo && b <= cut.b_hi) || b == cut.k_bin)) return;
       const uint32_t at = atomicAdd(&sh.list_n, 1u);
+      const int a = sh.anchor[col / kSlice];
       if (at < (uint32_t)kListCap)
-        sh.list[at] = Entry{composite(order_key(l), col), (double)__uint_as_float(bits - shift)};
+        sh.list[at] = Entry{composite(order_key(l), col),
+                            ldexp((double)mass_of(l, rule.c, (float)a), a - cut.anchor)};
     };
     // only the slices that hold such tokens: a top-k cut's bin holds a few, in as many slices
     uint64_t left = slices_with(v, r, cut, sh);
