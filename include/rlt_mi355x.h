@@ -280,10 +280,10 @@ int rlt_row_mass_f32(const float* x, int64_t rows, int64_t vocab, float* out, vo
  * Workspace (optional): with rlt_probabilities_workspace_size(n, 0, vocab) bytes, a
  * call that filters no row (max_top_k == 0, apply_top_p == 0) runs the row-split
  * form: each row spread over several workgroups (slice max and mass, then the
- * normalized slices; two launches).  Filtering calls on rows past 49152 columns (at
- * most 64 rows, or more than 81920 columns) run a row-split form of their own (three
- * launches).  Otherwise (workspace == NULL or smaller) one workgroup per row in one
- * launch.  The forms give the same values up to the rounding of the token masses and
+ * normalized slices; two launches).  Filtering calls on rows of more than 81920
+ * columns run a row-split form of their own (three launches).  Otherwise (fewer columns,
+ * or workspace == NULL or smaller) one workgroup per row in one launch.  A row's bits do
+ * not depend on the other rows of the call or their number.  The forms give the same values up to the rounding of the token masses and
  * their total; a top-p cut can differ only where the mass before a token equals the
  * threshold within that rounding.
  */

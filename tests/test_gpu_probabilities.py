@@ -661,6 +661,24 @@ def test_split_form_is_batch_invariant(pkg, dev):
         assert torch.equal(small.view(torch.int32), big[idx].view(torch.int32)), rows
 
 
+@pytest.mark.parametrize("vocab", [49153, 65536, 65537, 81920, 81921])
+def test_filtered_rows_are_batch_invariant(pkg, dev, vocab):
+    """A filtered row's form follows from its vocabulary: the same bits in batches of 1, 4,
+    64, 65 and 160 rows (a draft step's q and the verify round's p of the same logits)."""
+    _say("filtered batch invariance", vocab)
+    g = torch.Generator().manual_seed(vocab)
+    n = 160
+    logits = (torch.randn(n, vocab, generator=g) * 3).to(dev)
+    t = torch.full((n,), 0.9, device=dev)
+    k = torch.tensor([-1, 50, 20, -1])[torch.arange(n) % 4].to(dev)
+    p = torch.tensor([0.9, 1.0, 0.8, 0.95, 1.0])[torch.arange(n) % 5].to(dev)
+    plan = {"max_top_k": 50, "apply_top_p": True}
+    big = pkg.batched_probabilities(logits, t, k, p, **plan)
+    for m in (1, 4, 64, 65):
+        few = pkg.batched_probabilities(logits[:m], t[:m], k[:m], p[:m], **plan)
+        assert torch.equal(few.view(torch.int32), big[:m].view(torch.int32)), m
+
+
 # ------------------------------------------------- row-split form of filtered rows
 
 def _filter_rows(n, vocab, dtype, g):
@@ -681,10 +699,13 @@ def _filter_rows(n, vocab, dtype, g):
 
 @pytest.mark.parametrize("kind", ["p", "k", "kp", "p99", "mixed"])
 @pytest.mark.parametrize("n,vocab,dtype", [
-    (8, 49153, torch.float32),     # the first vocabulary of the form, rows on odd addresses
-    (64, 57344, torch.bfloat16),   # whole slices, the most rows below 81921 columns
+    (8, 49153, torch.float32),     # (one workgroup per row: the same distributions)
+    (64, 57344, torch.bfloat16),
     (6, 65536, torch.float16),
-    (70, 81921, torch.float32),    # one column past whole slices, more rows than 64
+    (6, 81920, torch.bfloat16),    # the last vocabulary below the form's
+    (70, 81921, torch.float32),    # the first of the form, rows on odd addresses, one column
+                                   # past whole slices
+    (64, 90112, torch.float16),    # whole slices
     (7, 151936, torch.bfloat16),
     (6, 262144, torch.float32),    # 32 slices
 ])

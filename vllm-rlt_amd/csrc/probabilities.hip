@@ -1505,13 +1505,16 @@ struct FilterPlan {
   int S;
 };
 
-// Rows that fit on one CU (65536 columns) and are enough to fill the chip are faster there:
-// top-p 0.9 of fp32 rows, one workgroup per row against this form, 160 rows of 49152: 27 / 38
-// us, of 65536: 39 / 47, of 100001: 89 / 71, of 151936: 150 / 80; 32 rows: 24 / 24, 31 / 26, 59
-// / 33, 91 / 34; 80 rows of 65537: 38 / 35, 160: 44 / 54.
-bool filter_plan(int64_t n_dist, int V, FilterPlan& p) {
+// By the vocabulary alone, so that a row's bits do not depend on its batch (a draft step's q
+// and the verify round's p of the same logits come from one form).  Past 81920 columns the
+// form is the faster one at every number of rows: top-p 0.9 of fp32 rows, one workgroup per row
+// against this form, 32 rows of 100001: 59 / 33 us, 160: 89 / 71; 32 of 151936: 91 / 34, 160:
+// 150 / 80.  Below, a row stays on one CU: few rows would gain here (32 of 65536: 31 / 26, of
+// 49152: 24 / 24; 80 of 65537: 38 / 35), enough rows to fill the chip lose (160 of 65536: 39 /
+// 47, of 65537: 44 / 54).
+bool filter_plan(int V, FilterPlan& p) {
   p.S = (V + filt::kSlice - 1) / filt::kSlice;
-  return V > 49152 && (n_dist <= 64 || V > 81920) && p.S <= filt::kMaxSlices;
+  return V > 81920 && p.S <= filt::kMaxSlices;
 }
 
 // Its workspace: slice statistics, histograms, row cuts.
@@ -1533,14 +1536,14 @@ struct FilterLayout {
 
 size_t filter_bytes(int64_t n_dist, int64_t n_arg, int V) {
   FilterPlan pl;
-  return n_dist > 0 && filter_plan(n_dist, V, pl) ? FilterLayout(pl, n_dist, n_arg).total : 0;
+  return n_dist > 0 && filter_plan(V, pl) ? FilterLayout(pl, n_dist, n_arg).total : 0;
 }
 
 // Whether a filtering call takes the form: the plan, and a workspace that holds it (other
 // calls run one workgroup per row).
 bool filter_form(int64_t n_dist, int64_t n_arg, int V, const void* ws, size_t ws_bytes,
                  FilterPlan& pl) {
-  return ws && n_dist > 0 && filter_plan(n_dist, V, pl) &&
+  return ws && n_dist > 0 && filter_plan(V, pl) &&
          ws_bytes >= FilterLayout(pl, n_dist, n_arg).total;
 }
 
