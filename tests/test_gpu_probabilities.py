@@ -755,6 +755,39 @@ def test_filter_form_matches_exact_distributions(pkg, dev, kind, n, vocab, dtype
     assert torch.equal(again[1:n - 1].view(torch.int32), got[1:n - 1].view(torch.int32))
 
 
+@pytest.mark.parametrize("vocab,dtype", [(81921, torch.float32), (90112, torch.float16),
+                                         (151936, torch.bfloat16), (262144, torch.float32)])
+def test_filter_form_cuts_below_a_slices_histogram(pkg, dev, vocab, dtype):
+    """Top-p cuts past the octaves that every slice's histogram holds: normal logits whose
+    peak's slice has little mass 16 octaves down, cuts 20 to 60 octaves down, slices without
+    any mass, against the float64 distribution and cut (tolerances as above)."""
+    _say("filter form deep", vocab, dtype)
+    g = torch.Generator().manual_seed(vocab)
+    p = torch.tensor([0.95, 0.99, 0.999, 0.9999, 0.99999, 1 - 2.0**-20]).repeat_interleave(3)
+    n = p.numel()
+    logits = torch.randn(n, vocab, generator=g) * torch.tensor([2.0, 3.0, 5.0]).repeat(6)[:, None]
+    logits[2, vocab - 1] += 25.0             # one slice far above the others
+    logits[4, 8192:16384] = -torch.inf
+    logits[7, :8192] -= 40.0
+    logits = logits.to(dtype)
+    t = torch.tensor([0.6, 0.8, 1.0])[torch.arange(n) % 3]
+    k = torch.full((n,), -1, dtype=torch.int64)
+    plan = {"max_top_k": 0, "apply_top_p": True}
+    got = pkg.batched_probabilities(logits.to(dev), t.to(dev), k.to(dev), p.to(dev), **plan).cpu()
+    for r in range(n):
+        x, order = (logits[r].double() / t[r].double()).sort(descending=True, stable=True)
+        e = (x - x[0]).exp()
+        before = (e.cumsum(0) - e) / e.sum()
+        kept = int((got[r] > 0).sum())
+        exact = max(1, int(((before <= float(p[r])) & (e > 0)).sum()))
+        lo, hi = min(kept, exact), max(kept, exact)
+        assert ((before[lo:hi] - float(p[r])).abs() <= EXACT_BAND).all(), f"row {r}: {kept} {exact}"
+        x = x.masked_fill(torch.arange(vocab) >= kept, -torch.inf)
+        want = torch.zeros(vocab, dtype=torch.float64).scatter_(0, order, x.softmax(0))
+        torch.testing.assert_close(got[r].double(), want, atol=ATOL, rtol=RTOL)
+        assert torch.equal(got[r] > 0, want > 0), f"row {r}"
+
+
 @pytest.mark.parametrize("vocab,dtype,flat", [(81921, torch.float32, False),
                                               (98304, torch.bfloat16, True)])
 def test_filter_form_in_verify_and_draft_calls(pkg, dev, vocab, dtype, flat):

@@ -41,11 +41,14 @@
 // float64 sums are exact in any order (so are an octave's).
 //
 // Depth.  A slice's histogram ends at octave 16 unless a cut may lie deeper: at 24 when the
-// mass below octave 16 exceeds half of the 1 - p that a top-p cut may drop, at 125 when the
+// mass below octave 16 exceeds a tenth of the 1 - p that a top-p cut may drop, at 125 when the
 // slice has fewer than k tokens in octaves 0 .. 16 (with k of them, the row's k-th token lies
-// there too).  Rows that this form does not decide -- a cut below a slice's histogram, more
-// tokens in the cut bins than the list holds (flat rows, large tie groups), logits out of
-// range -- run the exact path (probs_exact.h) in the second launch.
+// there too).  Slices decide that alone, so a row's top-p cut can still lie below the histogram
+// of one of them (its peak's slice holds little mass below octave 16, the others much): the row
+// launch then reads the row and bins what lies past the octaves that all slices hold
+// (deep_cut).  Rows that this form does not decide -- more tokens in the cut bins than the list
+// holds (flat rows, large tie groups), logits out of range -- run the exact path
+// (probs_exact.h) in the second launch.
 //
 // The order of tokens is the single-workgroup form's: logit descending, column ascending.
 // Included inside probabilities.hip's anonymous namespace.
@@ -65,6 +68,7 @@ constexpr int kShallow = 16;         // last octave of the usual histogram
 constexpr int kFineBins = 64, kCoarseBins = 4;
 constexpr int kBins = kFine * kFineBins + (kOctaves - kFine) * kCoarseBins;
 constexpr int kListCap = 2048;       // listed tokens per row
+constexpr int kDeepBins = 2048;      // steps that deep_cut bins: 32 octaves
 constexpr int kRowThreads = 1024;    // the row launch
 constexpr int kRowWaves = kRowThreads / RLT_WAVE;
 constexpr float kMaxScaled = 1048576.f;  // |l c| of a slice's maximum: 2^20
@@ -84,15 +88,18 @@ struct Hist {
   uint32_t cnt[kBins];
 };
 
-enum State { kNanRow = 0, kUnfiltered = 1, kCut = 2, kExact = 3 };
+// kDeep: only inside the row launch
+enum State { kNanRow = 0, kUnfiltered = 1, kCut = 2, kExact = 3, kDeep = 4 };
 
 // What the row launch found.
 struct RowCut {
   int32_t state;
   int32_t anchor;
   // bins [b_lo, b_hi] hold the last cut (their tokens are listed): earlier bins are kept,
-  // later ones dropped.  k_bin: the bin of the top-k cut (listed too), or -1
+  // later ones dropped; kBins + f: step f alone (deep_cut).  k_bin: the bin of the top-k cut
+  // (listed too), or -1
   int32_t b_lo, b_hi, k_bin;
+  int32_t reach;           // (kDeep) last octave that every slice's histogram holds
   uint32_t k_cnt_before;   // tokens before k_bin
   double mass_before;      // mass before b_lo
   double k_mass_before;    // mass before k_bin
@@ -436,7 +443,7 @@ __global__ __launch_bounds__(kThreads, 4) void rlt_filter_slice_kernel(
       top += sh.top_mass[i];
       n_top += sh.top_cnt[i];
     }
-    if (rule.do_p && z - top > 0.5 * (1.0 - (double)rule.p) * z) depth = kFine - 1;
+    if (rule.do_p && z - top > 0.1 * (1.0 - (double)rule.p) * z) depth = kFine - 1;
     if (rule.do_k && n_top < rule.kk) depth = kOctaves - 1;
     if (depth > kShallow) {  // uniform over the workgroup
       add(kShallowSteps, (depth + 1) * kFineBins, std::true_type{}, std::false_type{});
@@ -477,7 +484,10 @@ struct Entry {
 struct RowShared {
   union {
     struct {
-      Entry list[kListCap];
+      union {
+        Entry list[kListCap];
+        double deep[kDeepBins];
+      };
       double m[kRowWaves][RLT_WAVE];
       uint32_t n[kRowWaves][RLT_WAVE];
       int anchor[kMaxSlices];
@@ -635,6 +645,17 @@ __device__ __forceinline__ Crossing find(const RowHist& h, double limit, uint32_
   return out;
 }
 
+// The logits of steps [f_lo, f_hi) of the row's anchor, widened by more than what the product
+// and this quotient round.
+__device__ __forceinline__ void step_range(RowCut& cut, const Rule& rule, int f_lo, int f_hi) {
+  const float slack = 1e-3f + 1e-6f * fabsf((float)cut.anchor);
+  auto edge = [&](int f) {  // upper edge of a step's l c
+    return (float)(cut.anchor + 1) - (float)f * (1.f / kFineBins);
+  };
+  cut.l_hi = (edge(f_lo) + slack) / rule.c;
+  cut.l_lo = (edge(f_hi) - slack) / rule.c;
+}
+
 // The row's cut bins from its slices (the whole workgroup; every lane returns the same, and
 // every branch is on the row's values, so all waves meet at every barrier).
 __device__ __forceinline__ RowCut row_cut(const View& v, const Rule& rule, int64_t r, bool src_ok,
@@ -644,6 +665,7 @@ __device__ __forceinline__ RowCut row_cut(const View& v, const Rule& rule, int64
   cut.state = kNanRow;
   cut.anchor = kNoAnchor;
   cut.b_lo = cut.b_hi = cut.k_bin = -1;
+  cut.reach = -1;
   cut.k_cnt_before = 0;
   cut.mass_before = cut.k_mass_before = cut.z = 0.0;
   cut.l_lo = cut.l_hi = 0.f;
@@ -695,7 +717,22 @@ __device__ __forceinline__ RowCut row_cut(const View& v, const Rule& rule, int64
   }
   if (rule.do_p) {
     const Crossing lo = find<true>(h, rule.limit(z_lo), 0);
-    if (lo.bin < 0) return cut;
+    if (lo.bin < 0) {
+      // (with top-k every slice reaches its cut, and this one lies before it)
+      if (rule.do_k) return cut;
+      int reach = lane < v.S ? min(shift, kOctaves) + st.depth : kOctaves;
+      for (int off = 32; off >= 1; off >>= 1) reach = min(reach, __shfl_xor(reach, off, RLT_WAVE));
+      if (reach >= kOctaves - 1) return cut;
+      for (int o = 0; o <= reach; o += RLT_WAVE) {
+        double m;
+        uint32_t n;
+        h.octave(o + lane, m, n);
+        cut.mass_before += lane_sum(o + lane <= reach ? m : 0.0);
+      }
+      cut.reach = reach;
+      cut.state = kDeep;
+      return cut;
+    }
     const Crossing hi = rule.do_k ? find<true>(h, rule.limit(z_hi), 0) : lo;
     if (hi.bin < 0) return cut;
     cut.b_lo = lo.bin;
@@ -703,14 +740,7 @@ __device__ __forceinline__ RowCut row_cut(const View& v, const Rule& rule, int64
     cut.mass_before = lo.mass_before;
   }
   cut.state = kCut;
-  // the logits of bins b_lo .. max(b_hi, k_bin), widened by more than what the product and
-  // this quotient round
-  const float slack = 1e-3f + 1e-6f * fabsf((float)anchor);
-  auto edge = [&](int bin) {  // upper edge of a bin's l c
-    return (float)(anchor + 1) - (float)first_step(bin) * (1.f / kFineBins);
-  };
-  cut.l_hi = (edge(cut.b_lo) + slack) / rule.c;
-  cut.l_lo = (edge(max(cut.b_hi, cut.k_bin) + 1) - slack) / rule.c;
+  step_range(cut, rule, first_step(cut.b_lo), first_step(max(cut.b_hi, cut.k_bin) + 1));
   return cut;
 }
 
@@ -722,6 +752,75 @@ __device__ __forceinline__ double block_sum(RowShared& sh, double x) {
   for (int i = 0; i < kRowWaves; ++i) x += sh.sum[i];
   __syncthreads();
   return x;
+}
+
+// The step of a top-p cut past octave cut.reach, which the slices' histograms do not all hold:
+// one pass over the row's logits bins the 32 octaves from there on by steps (as much of a row
+// as a float32 top-p below 1 can cut: 2^18 tokens past them have less than 2^-30 of its mass).
+// Returns the cut at that step, or kExact.
+//
+// What bounds it: one CU's reads of the row and the LDS additions of the binned tokens, 15 to 30
+// us of the rows that need it, where the exact path took 300 to 700: 160 rows of 151936, T = 1,
+// logits of deviation 3, top-p 0.95: 704 -> 116 us (one workgroup per row: 212); 64 of 100003, T
+// = 0.6, top-p 0.99: 360 -> 45 (58).  Slices that go to octave 24 already for a tenth of the
+// droppable mass below octave 16 keep most rows out of it (for half of it the last case took 64,
+// and no other case less than 3% less).
+template <int DT, bool kVec>
+__device__ __forceinline__ void deep_cut(const char* __restrict__ src, int V, const Rule& rule,
+                                         RowShared& sh, RowCut& cut) {
+  const int t = threadIdx.x, w = t >> 6, lane = t & 63;
+  const int base = (cut.reach + 1) * kFineBins;
+  __syncthreads();
+  for (int i = t; i < kDeepBins; i += kRowThreads) sh.deep[i] = 0.0;
+  if (t == 0) sh.list_n = kDeepBins;
+  __syncthreads();
+  constexpr int Q = 8;  // loads in flight (four columns each); two per slice
+  static_assert(kSlice == 2 * 4 * kRowThreads && Q % 2 == 0, "two loads of the workgroup cover a slice");
+  for (int s0 = 0; s0 * kSlice < V; s0 += Q / 2) {
+    float x[Q][4];
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+      load_quad<DT, kVec>(src, (uint32_t)s0 * kSlice + 4 * (kRowThreads * q + t), V, x[q]);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int s = s0 + q / 2;
+      const int a = __builtin_amdgcn_readfirstlane(s * kSlice < V ? sh.anchor[s] : kNoAnchor);
+      if (a != kNoAnchor) {  // uniform: the slice has mass
+        const double unit = ldexp(1.0, a - cut.anchor);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int f = step_of(x[q][k], rule.c, cut.anchor) - base;
+          if ((uint32_t)f < (uint32_t)kDeepBins)
+            atomicAdd(&sh.deep[f], unit * (double)mass_of(x[q][k], rule.c, (float)a));
+        }
+      }
+    }
+  }
+  __syncthreads();
+  // the first step whose cumulative mass exceeds the limit: two steps a thread
+  const double limit = rule.limit(cut.z);
+  const double d0 = sh.deep[2 * t], d1 = sh.deep[2 * t + 1];
+  const double own = lane_scan(d0 + d1);
+  if (lane == 63) sh.sum[w] = own;
+  __syncthreads();
+  double before = cut.mass_before;
+  for (int i = 0; i < w; ++i) before += sh.sum[i];
+  before += own - (d0 + d1);
+  const int first = before + d0 > limit ? 2 * t : before + d0 + d1 > limit ? 2 * t + 1 : kDeepBins;
+  if (first < kDeepBins) atomicMin(&sh.list_n, (uint32_t)first);
+  __syncthreads();
+  const int at = (int)sh.list_n;
+  if (first == at && at < kDeepBins) sh.m[0][0] = at & 1 ? before + d0 : before;
+  __syncthreads();
+  cut.state = kExact;
+  if (at < kDeepBins) {
+    const int f = base + at;
+    cut.state = kCut;
+    cut.mass_before = sh.m[0][0];
+    cut.b_lo = cut.b_hi = kBins + f;
+    step_range(cut, rule, f, f + 1);
+  }
+  __syncthreads();
 }
 
 // Bin of a listed token, from its logit.
@@ -909,14 +1008,17 @@ __global__ __launch_bounds__(kRowThreads) void rlt_filter_row_kernel(
   const char* src = (const char*)logits + src_r * row_stride * (DT == RLT_F32 ? 4 : 2);
   const Rule rule(flt, r, V);
   RowCut cut = row_cut(v, rule, r, src_ok, sh);
+  if (cut.state == kDeep) deep_cut<DT, kVec>(src, V, rule, sh, cut);  // uniform
   if (t == 0) sh.list_n = 0;
   __syncthreads();
   if (cut.state == kCut) {
+    const bool deep = cut.b_lo >= kBins;
     // the tokens of the cut bins (a look at the logit first), each with the mass that its own
     // slice's histogram counted
     auto look = [&](float l, uint32_t col) {
       if (!(l >= cut.l_lo && l <= cut.l_hi)) return;
-      const int b = bin_of_step(step_of(l, rule.c, cut.anchor));
+      const int f = step_of(l, rule.c, cut.anchor);
+      const int b = deep ? kBins + f : bin_of_step(f);
       if (!((b >= cut.b_lo && b <= cut.b_hi) || b == cut.k_bin)) return;
       const uint32_t at = atomicAdd(&sh.list_n, 1u);
       const int a = sh.anchor[col / kSlice];
