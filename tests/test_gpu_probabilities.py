@@ -788,6 +788,23 @@ def test_filter_form_cuts_below_a_slices_histogram(pkg, dev, vocab, dtype):
         assert torch.equal(got[r] > 0, want > 0), f"row {r}"
 
 
+@pytest.mark.parametrize("vocab,dtype", [(81921, torch.float32), (151936, torch.bfloat16)])
+def test_filter_form_normalizes_beyond_float32(pkg, dev, vocab, dtype):
+    """A row's normalization adds no rounding of its own.  Over near-flat rows (no token has
+    1% of the mass) the values' own roundings, 2.5e-8 rms, average out of the row's sum: what
+    is left of sum - 1 is the common factor's error, 2.5e-8 rms if that is rounded to float32,
+    far below the bound if it is not."""
+    _say("filter form rounding", vocab, dtype)
+    g = torch.Generator().manual_seed(vocab)
+    n = 64
+    logits = torch.randn(n, vocab, generator=g).to(dtype)
+    got = pkg.batched_probabilities(
+        logits.to(dev), torch.ones(n, device=dev), torch.full((n,), -1, device=dev),
+        torch.full((n,), 0.9, device=dev), max_top_k=0, apply_top_p=True).cpu().double()
+    assert float(got.max()) < 0.01
+    assert float((got.sum(1) - 1).square().mean().sqrt()) <= 1e-8
+
+
 @pytest.mark.parametrize("vocab,dtype,flat", [(81921, torch.float32, False),
                                               (98304, torch.bfloat16, True)])
 def test_filter_form_in_verify_and_draft_calls(pkg, dev, vocab, dtype, flat):
