@@ -1181,6 +1181,33 @@ def test_long_window_store_ragged_rows(kernel, pkg, dev, kv, d, hkv):
         assert all(torch.equal(a, b) for a, b in zip(scales, want_scales))
 
 
+def test_window_store_of_many_padded_windows(kernel, pkg, dev):
+    """A ragged batch whose longest window could hold 2^20 rows: the padded windows take 2^24
+    workgroups of the store ahead of the prefill tiling, more than one grid of 256 threads
+    holds.  Exactly store_kv's bits in the pool, and the attention of a call with the windows'
+    own longest length."""
+    _say("padded window store")
+    g = torch.Generator().manual_seed(64)
+    n, bs, hkv, d, dtype = 64, 16, 8, 128, torch.bfloat16
+    q_lens = [65 if s % 7 else 1 for s in range(n)]
+    lengths = [w + 3 * s for s, w in enumerate(q_lens)]
+    pages = sum(-(-x // bs) for x in lengths) + 1
+    tables = random_tables(lengths, bs, pages, g)
+    rows = sum(q_lens)
+    q, k_new, v_new = (torch.randn(rows, hkv, d, generator=g).to(dtype).to(dev) for _ in range(3))
+    pools = [torch.randn(pages, bs, hkv, d, generator=g).to(dtype).to(dev) for _ in range(2)]
+    want = [x.clone() for x in pools]
+    seq = torch.repeat_interleave(torch.arange(n), torch.tensor(q_lens))
+    pos = torch.cat([torch.arange(c - w, c) for c, w in zip(lengths, q_lens)])
+    pkg.store_kv(*want, k_new, v_new, tables.long()[seq, pos // bs].to(dev), (pos % bs).to(dev))
+    cu = torch.tensor([0] + torch.cumsum(torch.tensor(q_lens), 0).tolist(), dtype=torch.int32)
+    args = (tables.to(dev), torch.tensor(lengths, dtype=torch.int32).to(dev), cu.to(dev))
+    out = kernel.prefill_store(q, k_new, v_new, *pools, *args, 1 << 20)
+    for got, ref in zip(pools, want):
+        assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+    assert torch.equal(out, kernel.prefill(q, *want, *args, max(q_lens)))
+
+
 @pytest.mark.parametrize("kv,d", [("same", 96), ("fp8_vector", 64), ("fp8_vector", 128)])
 def test_full_rounds_of_neighbouring_heads_equal_single_rows(kernel, dev, kv, d):
     """Batches that fill the persistent workgroups' rounds and whose heads share cache

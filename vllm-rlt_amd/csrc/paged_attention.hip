@@ -1535,6 +1535,9 @@ template <int D>
 constexpr int store_lanes() { return D <= 64 ? 8 : 16; }
 template <int D>
 constexpr int store_vectors() { return kStoreThreads / store_lanes<D>() * kStoreDepth; }
+// Workgroups of one launch: a grid holds fewer than 2^32 threads, and a call may ask for more
+// (its windows are padded to the longest).
+constexpr int64_t kStoreGrid = (int64_t)1 << 23;
 
 // NaN-propagating maximum over a group of L (8 or 16) lanes, in every lane.
 template <int L>
@@ -1551,12 +1554,14 @@ __device__ __forceinline__ float group_nan_max(float x) {
 }
 
 template <int QT, int KVT, int D, int SM>
-__global__ __launch_bounds__(kStoreThreads) void rlt_window_store_kernel(AttnParams P, int per_seq) {
+__global__ __launch_bounds__(kStoreThreads) void rlt_window_store_kernel(AttnParams P, uint32_t per_seq,
+                                                                         uint32_t first_wg) {
   constexpr int LPV = store_lanes<D>();
   constexpr int kPieces = D / 8;  // 16-byte pieces of a vector
   constexpr int kAtOnce = kStoreThreads / LPV;
-  const int seq = (int)(blockIdx.x / (unsigned)per_seq);
-  const int64_t first = (int64_t)(blockIdx.x - (unsigned)seq * per_seq) * store_vectors<D>();
+  const uint32_t wg = first_wg + blockIdx.x;
+  const int seq = (int)(wg / per_seq);
+  const int64_t first = (int64_t)(wg - seq * per_seq) * store_vectors<D>();
   const SeqView sv = seq_view(P, seq);
   const uint32_t vectors = 2 * P.hkv;  // of one row
   const int row0 = (int)(first / vectors);
@@ -1705,10 +1710,12 @@ int launch_vec_q(const AttnParams& P, int kv_dtype, dim3 grid, hipStream_t strea
 template <int QT, int KVT, int D, int SM>
 void launch_prefill_sm(const AttnParams& P, dim3 grid, int max_q, hipStream_t stream) {
   if (P.new_k) {
-    // (attention_impl bounds the product)
     const int64_t per_seq = ((int64_t)max_q * 2 * P.hkv + store_vectors<D>() - 1) / store_vectors<D>();
-    rlt_window_store_kernel<QT, KVT, D, SM><<<(unsigned)(P.num_seqs * per_seq), kStoreThreads, 0, stream>>>(
-        P, (int)per_seq);
+    const int64_t wgs = P.num_seqs * per_seq;  // (attention_impl: below 2^32)
+    for (int64_t at = 0; at < wgs; at += kStoreGrid)
+      rlt_window_store_kernel<QT, KVT, D, SM>
+          <<<(unsigned)(wgs - at < kStoreGrid ? wgs - at : kStoreGrid), kStoreThreads, 0, stream>>>(
+              P, (uint32_t)per_seq, (uint32_t)at);
   }
   // blocks of whole 16-position groups, and lane offsets within a group that fit 32 bits
   const int64_t most = (int64_t)1 << 26;
@@ -1921,8 +1928,9 @@ int attention_impl(const void* q, int64_t q_row_stride, int64_t q_head_stride,
       const int64_t wgs = (int64_t)num_seqs * P.rowgroups * num_kv_heads;
       if (wgs >= ((int64_t)1 << 31)) return RLT_ERR_UNSUPPORTED;
       const dim3 grid((unsigned)wgs);
-      // the window store's workgroups (at least 64 vectors each, two per row and kv head)
-      const int64_t swgs = (int64_t)num_seqs * num_kv_heads * (((int64_t)max_q_len + 31) / 32);
+      // the window store's workgroups: 64 vectors or more each, two vectors per row and kv
+      // head, so at most twice this many
+      const int64_t swgs = (int64_t)num_seqs * num_kv_heads * (((int64_t)max_q_len + 63) / 64);
       if (swgs >= ((int64_t)1 << 31)) return RLT_ERR_UNSUPPORTED;
       const bool fp8 = kv_dtype == RLT_FP8_E4M3;
       if (q_dtype == RLT_BF16) {
