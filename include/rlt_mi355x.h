@@ -277,16 +277,24 @@ int rlt_row_mass_f32(const float* x, int64_t rows, int64_t vocab, float* out, vo
  * kept); then softmax over the kept set.  max_top_k and apply_top_p are the host
  * plan's values, as in the reference.  Rows holding NaN (or with a non-finite
  * max) are written as NaN.  V <= 262144.
- * Workspace (optional): with rlt_probabilities_workspace_size(n, 0, vocab) bytes, a
- * call that filters no row (max_top_k == 0, apply_top_p == 0) runs the row-split
+ * Workspace (optional): with rlt_probabilities_plan_workspace_size(n, 0, vocab, max_top_k,
+ * apply_top_p) bytes, a call that filters no row (max_top_k == 0, apply_top_p == 0) runs the row-split
  * form: each row spread over several workgroups (slice max and mass, then the
  * normalized slices; two launches).  Filtering calls on rows of more than 81920
- * columns run a row-split form of their own (three launches).  Otherwise (fewer columns,
+ * columns run a row-split form of their own (three launches for up to 256 MiB of
+ * histograms, 25 KB per 8192 columns of a row; further rows in further launches, through the
+ * same memory).  Otherwise (fewer columns,
  * or workspace == NULL or smaller) one workgroup per row in one launch.  A row's bits do
  * not depend on the other rows of the call or their number.  The forms give the same values up to the rounding of the token masses and
  * their total; a top-p cut can differ only where the mass before a token equals the
  * threshold within that rounding.
+ * The plan queries give the bytes of a call with these filters (0: none needed); the queries
+ * without a plan give the largest of any call's, so 256 MiB and more for many rows of more
+ * than 81920 columns, where a call that filters no row needs 16 bytes per 4096 columns of one.
  */
+size_t rlt_probabilities_plan_workspace_size(int64_t rows, int64_t argmax_rows, int64_t vocab,
+                                             int64_t max_top_k, int32_t apply_top_p);
+
 size_t rlt_probabilities_workspace_size(int64_t rows, int64_t argmax_rows, int64_t vocab);
 
 int rlt_batched_probabilities(const void* logits, int32_t logits_dtype, int64_t row_stride,
@@ -302,13 +310,18 @@ int rlt_batched_probabilities(const void* logits, int32_t logits_dtype, int64_t 
  * with temperature[j] / top_k[j] / top_p[j], and proposed[random_rows[j]] =
  * categorical(q_out row j, u[j]) (0 for an invalid row).  Replaces the draft step
  * of vllm_rlt/worker/async_speculative.py:645-663 (argmax, _probabilities on
- * logits[random_rows], categorical, proposed[random_rows] = sampled) in three
- * launches without host synchronization.  q_out rows are q_stride floats apart (pass
- * the q[:, offset] view).  Workspace: rlt_propose_drafts_workspace_size(m, r, vocab)
- * (row-split distributions when no row is filtered), or at least
- * rlt_categorical_workspace_size(r, vocab) (one workgroup per row).
+ * logits[random_rows], categorical, proposed[random_rows] = sampled) without host
+ * synchronization: the distribution launches (one workgroup per row: one, row-split as in
+ * rlt_batched_probabilities: two or three) and the draws' (two, or one after the row-split
+ * forms, which write the draws' tile totals).  q_out rows are q_stride floats apart (pass
+ * the q[:, offset] view).  Workspace: rlt_propose_drafts_plan_workspace_size(m, r, vocab,
+ * max_top_k, apply_top_p), which selects rlt_batched_probabilities' form for these filters,
+ * or at least rlt_categorical_workspace_size(r, vocab) (one workgroup per row).
  * A random row index outside [0, m) gives an all-NaN q_out row and proposes nothing.
  */
+size_t rlt_propose_drafts_plan_workspace_size(int64_t m, int64_t r, int64_t vocab,
+                                              int64_t max_top_k, int32_t apply_top_p);
+
 size_t rlt_propose_drafts_workspace_size(int64_t m, int64_t r, int64_t vocab);
 
 int rlt_propose_drafts(const void* logits, int32_t logits_dtype, int64_t row_stride, int64_t m,
@@ -323,13 +336,13 @@ int rlt_propose_drafts(const void* logits, int32_t logits_dtype, int64_t row_str
  * maximal column, NaN the maximum) and, for the random rows random_rows[j] (j < r),
  * p_out row j = batched_probabilities of that logits row with temperature[j] /
  * top_k[j] / top_p[j] (rows p_stride floats apart, e.g. a p[ranks, offsets] view when
- * rows line up).  One launch: the argmax rows are extra workgroups of the
- * distribution launch.  Replaces vllm_rlt/worker/async_speculative.py:678-692
+ * rows line up).  The argmax rows are extra workgroups of the first distribution launch
+ * (the only one, with one workgroup per row).  Replaces vllm_rlt/worker/async_speculative.py:678-692
  * (target = logits.argmax(-1); p[v_ranks, v_offsets] = _probabilities(logits[v_rows],
  * ...)).  A random row index outside [0, m) gives an all-NaN p row.  Workspace:
- * rlt_probabilities_workspace_size(r, m, vocab) bytes (row-split form for calls
- * that filter no row, the argmax rows as extra slices), or NULL (one workgroup per
- * row).
+ * rlt_probabilities_plan_workspace_size(r, m, vocab, max_top_k, apply_top_p) bytes
+ * (rlt_batched_probabilities' form for these filters, the argmax rows as extra slices), or
+ * NULL (one workgroup per row).
  */
 int rlt_verify_distributions(const void* logits, int32_t logits_dtype, int64_t row_stride,
                              int64_t m, int64_t vocab, const int64_t* random_rows, int64_t r,
@@ -344,13 +357,14 @@ int rlt_verify_distributions(const void* logits, int32_t logits_dtype, int64_t r
  * (temperature / top_k / top_p per row), then speculative_accept with p_out.  Bitwise
  * the results of rlt_verify_distributions (all rows random) followed by
  * rlt_speculative_accept; the draft rows' float32 row-sum partials are computed by
- * otherwise idle workgroups of the distribution launch, so the acceptance then sums
- * only p.  Replaces vllm_rlt/worker/async_speculative.py:678-692 (_verify) followed by
- * :727-734 (speculative_accept).  Workspace: rlt_verify_accept_workspace_size
- * (row-split distributions when no row is filtered, the draft rows' partials as
- * extra workgroups of its first launch), or at least
+ * otherwise idle workgroups of the first distribution launch, and p's with its rows.  Replaces vllm_rlt/worker/async_speculative.py:678-692 (_verify) followed by
+ * :727-734 (speculative_accept).  Workspace: rlt_verify_accept_plan_workspace_size
+ * (rlt_batched_probabilities' form for these filters), or at least
  * rlt_speculative_accept_workspace_size (one workgroup per row).
  */
+size_t rlt_verify_accept_plan_workspace_size(int64_t n, int32_t w1, int64_t vocab,
+                                             int64_t max_top_k, int32_t apply_top_p);
+
 size_t rlt_verify_accept_workspace_size(int64_t n, int32_t w1, int64_t vocab);
 
 int rlt_verify_accept(const void* target_logits, int32_t logits_dtype, int64_t row_stride,

@@ -56,6 +56,33 @@ def test_workspace_queries_are_host_only(pkg):
     assert lib.rlt_paged_attention_uses_prefill(2, 2, 256, 512) == 0
 
 
+def test_workspace_queries_of_a_plan(pkg):
+    """A call's own size: what its filters need, histograms of row-split filters bounded at
+    256 MiB (plus statistics and cuts, under 1 KB a slice), and never more than the queries
+    without a plan give."""
+    from vllm_rlt_amd import _lib
+
+    lib = _lib.library()
+    size = lib.rlt_probabilities_plan_workspace_size
+    assert size(640, 0, 151936, 0, 0) < 1 << 20       # unfiltered: block statistics
+    assert size(64, 0, 81920, 50, 1) == 0             # one workgroup per row
+    for rows, vocab in ((1, 81921), (640, 151936), (2000, 262144), (1, 262144)):
+        slices = rows * -(-vocab // 8192)
+        for plan in ((50, 0), (0, 1), (50, 1)):
+            assert slices * 24 < size(rows, 0, vocab, *plan) <= (256 << 20) + slices * 1024
+            assert size(rows, rows, vocab, *plan) > size(rows, 0, vocab, *plan)
+            assert lib.rlt_probabilities_workspace_size(rows, 0, vocab) >= size(rows, 0, vocab, *plan)
+    assert size(5, 0, 262145, 0, 1) == size(5, 0, 262145, 0, 0) == size(-1, 0, 9, 0, 0) == 0
+    assert lib.rlt_probabilities_workspace_size(9, 0, 81920) == size(9, 0, 81920, 0, 0)
+    accept, draft = lib.rlt_speculative_accept_workspace_size, lib.rlt_categorical_workspace_size
+    both = (lib.rlt_verify_accept_plan_workspace_size, lib.rlt_propose_drafts_plan_workspace_size)
+    assert both[0](128, 4, 151936, 0, 0) - accept(128, 4, 151936) < 1 << 20
+    assert both[1](640, 640, 151936, 0, 0) - draft(640, 151936) < 2 << 20
+    assert both[0](128, 4, 151936, 0, 1) > both[0](128, 4, 151936, 0, 0)
+    assert both[1](640, 640, 151936, 9, 0) > both[1](640, 640, 151936, 0, 0)
+    assert both[1](640, 0, 151936, 9, 0) == 0
+
+
 def test_argument_errors_return_status_without_launching(pkg):
     from vllm_rlt_amd import _lib
 

@@ -805,6 +805,71 @@ def test_filter_form_normalizes_beyond_float32(pkg, dev, vocab, dtype):
     assert float((got.sum(1) - 1).square().mean().sqrt()) <= 1e-8
 
 
+def test_filter_form_in_groups_of_rows(pkg, dev):
+    """Rows past the histograms' 256 MiB go in groups (of 256 rows of 262144 columns): the bits
+    of smaller calls, argmax rows and rows outside the logits included."""
+    _say("filter form groups")
+    g = torch.Generator(device=dev).manual_seed(17)
+    m, r, vocab = 301, 300, 262144
+    logits = (torch.randn(m, vocab, generator=g, device=dev) * 3).bfloat16()
+    rows = torch.randperm(m, generator=g, device=dev)[:r]
+    rows[[0, 255, 256]] = torch.tensor([m, -1, m + 5], device=dev)
+    t = torch.full((r,), 0.8, device=dev)
+    k = torch.tensor([-1, 50], device=dev).repeat(150)
+    p = torch.tensor([0.9, 1.0, 0.95], device=dev).repeat(100)
+    plan = {"max_top_k": 50, "apply_top_p": True}
+    target, got = pkg.verify_distributions(logits, rows, t, k, p, **plan)
+    assert torch.equal(target, logits.float().argmax(-1))
+    for part in (slice(0, 100), slice(200, 300)):
+        few = pkg.verify_distributions(logits, rows[part], t[part], k[part], p[part], **plan)[1]
+        assert torch.equal(few.view(torch.int32), got[part].view(torch.int32))
+    assert bool(got[[0, 255, 256]].isnan().all()) and not bool(got[1:255].isnan().any())
+    u = torch.rand(r, generator=g, device=dev)
+    proposed, q = pkg.propose_drafts(logits, rows, t, k, p, u, **plan)
+    assert torch.equal(q.view(torch.int32), got.view(torch.int32))
+    ok = (rows >= 0) & (rows < m)
+    want = target.clone()
+    want[rows[ok]] = pkg.categorical(q[ok].contiguous(), u[ok])[0]
+    assert torch.equal(proposed, want)
+    # the acceptance's row sums of every group (260 rows: 256 and 4)
+    n, w1 = 52, 4
+    every = torch.arange(n * (w1 + 1), device=dev)
+    target, p_rows = pkg.verify_distributions(logits, every, t[:260], k[:260], p[:260], **plan)
+    p_rows = p_rows.view(n, w1 + 1, vocab)
+    draft = p_rows[:, :w1].argmax(-1)
+    args = (draft, torch.full((n,), w1, device=dev), p_rows[:, :w1].roll(1, 0).contiguous(),
+            torch.rand(n, w1, generator=g, device=dev), torch.rand(n, generator=g, device=dev))
+    target_a, p_a, res = pkg.verify_accept(logits[:260].view(n, w1 + 1, vocab), t[:260], k[:260],
+                                           p[:260], *args, **plan)
+    want = pkg.speculative_accept(*args[:3], p_rows, *args[3:])
+    assert torch.equal(target_a.view(-1), target[:260])
+    assert torch.equal(p_a.view(torch.int32), p_rows.view(torch.int32))
+    assert all(torch.equal(a, b) for a, b in zip(res, want))
+
+
+def test_calls_allocate_what_their_filters_need(pkg, dev):
+    """An unfiltered call on a long vocabulary takes no histograms: 64 rows of 151936 (31 MB of
+    them for a filtering call) allocate their outputs and under 1 MiB more."""
+    _say("unfiltered workspace")
+    n, vocab = 64, 151936
+    logits = torch.randn(n, vocab, device=dev)
+    t, p = torch.ones(n, device=dev), torch.ones(n, device=dev)
+    k = torch.full((n,), -1, device=dev)
+    rows = torch.arange(n, device=dev)
+    plan = {"max_top_k": 0, "apply_top_p": False}
+
+    def extra(call):
+        call()
+        torch.cuda.reset_peak_memory_stats(dev)
+        before = torch.cuda.memory_allocated(dev)
+        call()
+        return torch.cuda.max_memory_allocated(dev) - before - n * vocab * 4
+
+    assert extra(lambda: pkg.batched_probabilities(logits, t, k, p, **plan)) < 1 << 20
+    assert extra(lambda: pkg.verify_distributions(logits, rows, t, k, p, **plan)) < 1 << 20
+    assert extra(lambda: pkg.propose_drafts(logits, rows, t, k, p, t, **plan)) < 1 << 20
+
+
 @pytest.mark.parametrize("vocab,dtype,flat", [(81921, torch.float32, False),
                                               (98304, torch.bfloat16, True)])
 def test_filter_form_in_verify_and_draft_calls(pkg, dev, vocab, dtype, flat):

@@ -1517,11 +1517,21 @@ bool filter_plan(int V, FilterPlan& p) {
   return V > 81920 && p.S <= filt::kMaxSlices;
 }
 
-// Its workspace: slice statistics, histograms, row cuts.
+// Its workspace: slice statistics, histograms, row cuts.  The histograms take 25 KB a slice,
+// more than the slice's own logits in 16 bits, so they are bounded: further rows go in groups,
+// one after the other, through the same memory.  A group is a multiple of 256 rows, the row
+// launch's workgroups at a time (two groups of 320 rows of 81921 columns took 194 us, 640 at
+// once 171).
+constexpr size_t kHistBytes = (size_t)256 << 20;
 struct FilterLayout {
   size_t hist, cuts, total;
+  int64_t group;  // rows of a group
   FilterLayout(const FilterPlan& pl, int64_t n_dist, int64_t n_arg) {
-    const size_t slices = (size_t)n_dist * pl.S;
+    // (at least 256: a row has at most 32 slices)
+    static_assert(kHistBytes / (filt::kMaxSlices * sizeof(filt::Hist)) >= 256, "one group");
+    const int64_t most = (int64_t)(kHistBytes / (pl.S * sizeof(filt::Hist))) / 256 * 256;
+    group = n_dist < most ? n_dist : most;
+    const size_t slices = (size_t)group * pl.S;
     size_t at = rlt_align_up((size_t)(n_dist + n_arg) * pl.S * sizeof(filt::SliceStat), 256);
     auto take = [&](size_t bytes) {
       const size_t here = at;
@@ -1547,7 +1557,7 @@ bool filter_form(int64_t n_dist, int64_t n_arg, int V, const void* ws, size_t ws
          ws_bytes >= FilterLayout(pl, n_dist, n_arg).total;
 }
 
-// The form's three launches (arguments as launch_split's).
+// The form's three launches per group of rows (arguments as launch_split's).
 template <int DT>
 void launch_filter(const FilterPlan& pl, int64_t n_dist, const void* logits, const int64_t* rows,
                      int64_t n_src, int64_t row_stride, int V, const filt::Filter& flt, float* out,
@@ -1576,21 +1586,27 @@ void launch_filter(const FilterPlan& pl, int64_t n_dist, const void* logits, con
   const cascade::RowGeom geo = cascade::row_geom(V);
   const int64_t per_block = filt::kThreads / cascade::kGroupThreads;
   const int64_t qm_blocks = qm_src ? (qm_rows * geo.groups + per_block - 1) / per_block : 0;
-  const unsigned g1 = (unsigned)((n_dist + v.n_arg) * pl.S + qm_blocks);
-  const unsigned g2 = (unsigned)(n_dist * pl.S);
-  const unsigned g3 = g2 + (unsigned)((v.n_arg + filt::kThreads - 1) / filt::kThreads);
   const dim3 b(filt::kThreads);
 #define RLT_FILTER_LAUNCH(VEC)                                                                  \
   filt::rlt_filter_slice_kernel<DT, VEC><<<g1, b, 0, stream>>>(                              \
       logits, rows, n_src, row_stride, V, flt, v, qm_src, qm_rows, qm_out);                     \
-  filt::rlt_filter_row_kernel<DT, VEC><<<(unsigned)n_dist, filt::kRowThreads, 0, stream>>>(     \
+  filt::rlt_filter_row_kernel<DT, VEC><<<(unsigned)v.row_n, filt::kRowThreads, 0, stream>>>(    \
       logits, rows, n_src, row_stride, V, flt, v, out, out_stride);                             \
   filt::rlt_filter_write_kernel<DT, VEC><<<g3, b, 0, stream>>>(                              \
       logits, rows, n_src, row_stride, V, flt, v, out, out_stride, out_vec)
-  if (vec) {
-    RLT_FILTER_LAUNCH(true);
-  } else {
-    RLT_FILTER_LAUNCH(false);
+  for (v.row0 = 0; v.row0 < n_dist; v.row0 += at.group) {
+    v.row_n = n_dist - v.row0 < at.group ? n_dist - v.row0 : at.group;
+    // (the argmax-only rows and the draft rows' partials go with the first group)
+    const bool first = v.row0 == 0;
+    if (!first) v.n_arg = 0;
+    const unsigned g1 = (unsigned)((v.row_n + v.n_arg) * pl.S + (first ? qm_blocks : 0));
+    const unsigned g3 =
+        (unsigned)(v.row_n * pl.S + (v.n_arg + filt::kThreads - 1) / filt::kThreads);
+    if (vec) {
+      RLT_FILTER_LAUNCH(true);
+    } else {
+      RLT_FILTER_LAUNCH(false);
+    }
   }
 #undef RLT_FILTER_LAUNCH
 }
@@ -1625,13 +1641,17 @@ int rlt_categorical_rows(const float* weights, int64_t w_stride, const float* u,
 
 extern "C" {
 
-size_t rlt_probabilities_workspace_size(int64_t rows, int64_t argmax_rows, int64_t vocab) {
+size_t rlt_probabilities_plan_workspace_size(int64_t rows, int64_t argmax_rows, int64_t vocab,
+                                             int64_t max_top_k, int32_t apply_top_p) {
   SplitPlan pl;
-  if (rows < 0 || argmax_rows < 0 || vocab < 1 || vocab > 0x7fffffff ||
-      !split_plan(rows, (int)vocab, pl))
-    return 0;
-  const size_t sp = split_bytes(rows, argmax_rows, (int)vocab);
-  const size_t ft = filter_bytes(rows, argmax_rows, (int)vocab);
+  if (rows < 0 || argmax_rows < 0 || vocab < 1 || vocab > 0x7fffffff) return 0;
+  if (max_top_k > 0 || apply_top_p) return filter_bytes(rows, argmax_rows, (int)vocab);
+  return split_plan(rows, (int)vocab, pl) ? split_bytes(rows, argmax_rows, (int)vocab) : 0;
+}
+
+size_t rlt_probabilities_workspace_size(int64_t rows, int64_t argmax_rows, int64_t vocab) {
+  const size_t sp = rlt_probabilities_plan_workspace_size(rows, argmax_rows, vocab, 0, 0);
+  const size_t ft = rlt_probabilities_plan_workspace_size(rows, argmax_rows, vocab, 0, 1);
   return sp > ft ? sp : ft;
 }
 
@@ -1711,9 +1731,16 @@ int rlt_greedy_accept(const int64_t* draft_tokens, const int64_t* drafts, const 
 }
 
 size_t rlt_propose_drafts_workspace_size(int64_t m, int64_t r, int64_t vocab) {
-  if (m < 0 || r < 0) return 0;
-  return rlt_align_up(r > 0 ? rlt_categorical_workspace_size(r, vocab) : 0, 256) +
-         (r > 0 ? rlt_probabilities_workspace_size(r, m, vocab) : 0);
+  if (m < 0 || r <= 0) return 0;
+  return rlt_align_up(rlt_categorical_workspace_size(r, vocab), 256) +
+         rlt_probabilities_workspace_size(r, m, vocab);
+}
+
+size_t rlt_propose_drafts_plan_workspace_size(int64_t m, int64_t r, int64_t vocab,
+                                              int64_t max_top_k, int32_t apply_top_p) {
+  if (m < 0 || r <= 0) return 0;
+  return rlt_align_up(rlt_categorical_workspace_size(r, vocab), 256) +
+         rlt_probabilities_plan_workspace_size(r, m, vocab, max_top_k, apply_top_p);
 }
 
 int rlt_propose_drafts(const void* logits, int32_t logits_dtype, int64_t row_stride, int64_t m,
@@ -1838,6 +1865,13 @@ size_t rlt_verify_accept_workspace_size(int64_t n, int32_t w1, int64_t vocab) {
   if (n < 0 || w1 < 0) return 0;
   return rlt_align_up(rlt_speculative_accept_workspace_size(n, w1, vocab), 256) +
          rlt_probabilities_workspace_size(n * (w1 + 1), 0, vocab);
+}
+
+size_t rlt_verify_accept_plan_workspace_size(int64_t n, int32_t w1, int64_t vocab,
+                                             int64_t max_top_k, int32_t apply_top_p) {
+  if (n < 0 || w1 < 0) return 0;
+  return rlt_align_up(rlt_speculative_accept_workspace_size(n, w1, vocab), 256) +
+         rlt_probabilities_plan_workspace_size(n * (w1 + 1), 0, vocab, max_top_k, apply_top_p);
 }
 
 int rlt_verify_accept(const void* target_logits, int32_t logits_dtype, int64_t row_stride,

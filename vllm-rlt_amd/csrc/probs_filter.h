@@ -113,10 +113,12 @@ struct RowCut {
 
 struct View {
   SliceStat* stats;     // [(n_dist + n_arg) S]
-  Hist* hist;           // [n_dist S]
+  Hist* hist;           // [row_n S]
   RowCut* cuts;         // [n_dist]
   int S;
   int64_t n_dist, n_arg;
+  // the launches' distribution rows: [row0, row0 + row_n) of the n_dist
+  int64_t row0, row_n;
   int64_t* targets;     // argmax outputs, or nullptr
   int fused;            // distribution row r's argmax goes to targets[r]
   int skip_drawn;       // argmax-only rows listed in rows[] are left to the draws
@@ -124,6 +126,8 @@ struct View {
   double* tile_sum;     // totals and flags of the written rows' 4096-column tiles, or nullptr
   uint32_t* tile_flags;
   int tiles;
+  // the S histograms of distribution row r
+  __device__ __forceinline__ Hist* row_hist(int64_t r) const { return hist + (r - row0) * S; }
 };
 
 struct Filter {
@@ -243,9 +247,8 @@ struct SliceShared {
   uint32_t top_cnt[kWaves];
 };
 
-// Workgroups [0, n_dist S): slices of the distribution rows (logits row rows[r], or r);
-// [n_dist S, (n_dist + n_arg) S): argmax-only slices of logits row r - n_dist; then the
-// draft rows' float32 row-sum partials of the acceptance sampler (eight 8192-float groups
+// Workgroups [0, row_n S): slices of distribution rows r = row0 + (logits row rows[r], or r);
+// then n_arg S: argmax-only slices of logits rows 0 .. n_arg - 1; then the draft rows' float32 row-sum partials of the acceptance sampler (eight 8192-float groups
 // per workgroup) when qm_src is set.
 template <int DT, bool kVec>
 __global__ __launch_bounds__(kThreads, 4) void rlt_filter_slice_kernel(
@@ -257,7 +260,7 @@ __global__ __launch_bounds__(kThreads, 4) void rlt_filter_slice_kernel(
     cascade::ChunkSums cs[kThreads / cascade::kGroupThreads];
   } lds;
   const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-  const int64_t n_slices = (v.n_dist + v.n_arg) * v.S;
+  const int64_t n_slices = (v.row_n + v.n_arg) * v.S;
   if ((int64_t)blockIdx.x >= n_slices) {
     const cascade::RowGeom geo = cascade::row_geom(V);
     const int sub = t / cascade::kGroupThreads, st = t % cascade::kGroupThreads;
@@ -279,9 +282,10 @@ __global__ __launch_bounds__(kThreads, 4) void rlt_filter_slice_kernel(
     return;
   }
   SliceShared& sh = lds.s;
-  const int64_t r = (int64_t)blockIdx.x / v.S;
+  const int64_t at = (int64_t)blockIdx.x / v.S;
   const int s = (int)((int64_t)blockIdx.x % v.S);
-  const bool dist = r < v.n_dist;
+  const bool dist = at < v.row_n;
+  const int64_t r = dist ? v.row0 + at : v.n_dist + at - v.row_n;
   SliceStat* stat = v.stats + r * v.S + s;
   if (!dist && v.skip_drawn && rows) {
     // an argmax-only row that is also drawn: an empty key, no logits read
@@ -408,7 +412,7 @@ __global__ __launch_bounds__(kThreads, 4) void rlt_filter_slice_kernel(
   for (int i = 0; i < kWaves; ++i) z += sh.z[i];  // fixed order
   int depth = kShallow;
   if (cuts) {
-    Hist* hist = v.hist + r * v.S + s;
+    Hist* hist = v.row_hist(r) + s;
     double top = 0.0;
     uint32_t n_top = 0;
     auto put = [&](int o) {  // a fine octave, by one wave
@@ -703,7 +707,7 @@ __device__ __forceinline__ RowCut row_cut(const View& v, const Rule& rule, int64
     cut.state = kUnfiltered;
     return cut;
   }
-  const RowHist h{v.hist + r * v.S, v.S, shift, st.depth, rule.do_k, &sh};
+  const RowHist h{v.row_hist(r), v.S, shift, st.depth, rule.do_k, &sh};
   double z_lo = z, z_hi = z;
   if (rule.do_k) {
     const Crossing k = find<false>(h, 0.0, (uint32_t)rule.kk);
@@ -985,7 +989,7 @@ __device__ __forceinline__ uint64_t slices_with(const View& v, int64_t r, const 
   bool held = s < v.S && sh.anchor[s] != kNoAnchor;
   if (held && cut.b_hi < kFine * kFineBins && cut.b_hi - cut.b_lo < 8 &&
       cut.k_bin < kFine * kFineBins) {
-    const double* mass = v.hist[r * v.S + s].mass;
+    const double* mass = v.row_hist(r)[s].mass;
     const int shift = (cut.anchor - sh.anchor[s]) * kFineBins;
     // (bins before the slice's first octave are empty)
     held = cut.k_bin >= shift && mass[cut.k_bin - shift] != 0.0;
@@ -1001,7 +1005,7 @@ __global__ __launch_bounds__(kRowThreads) void rlt_filter_row_kernel(
     int64_t row_stride, int V, Filter flt, View v, float* __restrict__ out, int64_t out_stride) {
   __shared__ RowShared sh;
   const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-  const int64_t r = blockIdx.x;
+  const int64_t r = v.row0 + blockIdx.x;
   int64_t src_r = rows ? rows[r] : r;
   const bool src_ok = src_r >= 0 && src_r < n_src;
   if (!src_ok) src_r = 0;
@@ -1189,7 +1193,7 @@ __global__ __launch_bounds__(kThreads) void rlt_filter_write_kernel(
     int out_vec) {
   __shared__ WriteShared sh;
   const int t = threadIdx.x;
-  const int64_t n_slices = v.n_dist * v.S;
+  const int64_t n_slices = v.row_n * v.S;
   if ((int64_t)blockIdx.x >= n_slices) {
     // argmax-only rows, one thread each; a row left to its draw has empty keys
     const int64_t i = ((int64_t)blockIdx.x - n_slices) * kThreads + t;
@@ -1201,7 +1205,7 @@ __global__ __launch_bounds__(kThreads) void rlt_filter_write_kernel(
     v.targets[i] = split::argmax_column(best);
     return;
   }
-  const int64_t r = (int64_t)blockIdx.x / v.S;
+  const int64_t r = v.row0 + (int64_t)blockIdx.x / v.S;
   const int s = (int)((int64_t)blockIdx.x % v.S);
   int64_t src_r = rows ? rows[r] : r;
   const bool src_ok = src_r >= 0 && src_r < n_src;

@@ -287,7 +287,7 @@ Tensor spec_probs(const Tensor& logits, const Tensor& temperature, const Tensor&
   const Tensor& p = need(top_p, at::kFloat, "top_p");
   const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
   // row-split form (several workgroups per row) when it applies to this vocabulary
-  const size_t nbytes = rlt_probabilities_workspace_size(n, 0, vocab);
+  const size_t nbytes = rlt_probabilities_plan_workspace_size(n, 0, vocab, max_top_k, apply_top_p);
   const Tensor ws = workspace(nbytes, x);
   const int status = rlt_batched_probabilities(
       ptr(x), dtype_code(x.scalar_type()), x.stride(0), n, vocab, (const float*)ptr(t),
@@ -414,7 +414,7 @@ std::tuple<Tensor, Tensor> verify_distributions(const Tensor& logits, const Tens
     p = need(top_p, at::kFloat, "top_p");
   }
   const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-  const size_t nbytes = r ? rlt_probabilities_workspace_size(r, m, vocab) : 0;
+  const size_t nbytes = r ? rlt_probabilities_plan_workspace_size(r, m, vocab, max_top_k, apply_top_p) : 0;
   const Tensor ws = workspace(nbytes, x);
   const int status = rlt_verify_distributions(
       ptr(x), dtype_code(x.scalar_type()), x.stride(0), m, vocab, (const int64_t*)ptr(rows), r,
@@ -467,7 +467,8 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> verify_accept(
   const Tensor& ua = need(u_accept, at::kFloat, "u_accept");
   const Tensor& uf = need(u_final, at::kFloat, "u_final");
   const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-  const Tensor ws = workspace(rlt_verify_accept_workspace_size(n, (int32_t)w1, vocab), x);
+  const Tensor ws = workspace(
+      rlt_verify_accept_plan_workspace_size(n, (int32_t)w1, vocab, max_top_k, apply_top_p), x);
   const int status = rlt_verify_accept(
       ptr(x), dtype_code(x.scalar_type()), x.stride(0), (const float*)ptr(t),
       (const int64_t*)ptr(k), (const float*)ptr(pp), max_top_k, apply_top_p ? 1 : 0,
