@@ -1181,6 +1181,42 @@ def test_long_window_store_ragged_rows(kernel, pkg, dev, kv, d, hkv):
         assert all(torch.equal(a, b) for a, b in zip(scales, want_scales))
 
 
+@pytest.mark.parametrize("kv", ["same", "fp8"])
+@pytest.mark.parametrize("stride", [(1 << 26) - 16, 1 << 26])
+def test_pools_of_long_token_strides(pkg, dev, kv, stride):
+    """Token strides at the line between 32-bit lane offsets within a tile and per-position
+    addresses: decode, windows, compensated windows and the prefill tiling give the bits of a
+    contiguous pool."""
+    _say("long token stride", kv, stride)
+    g = torch.Generator().manual_seed(26)
+    blocks, bs, hkv, hq, d = 6, 16, 2, 4, 64
+    k, v = (torch.randn(blocks, bs, hkv, d, generator=g).to(torch.bfloat16) for _ in range(2))
+    scales = ()
+    if kv == "fp8":
+        k, v = k.to(torch.float8_e4m3fn), v.to(torch.float8_e4m3fn)
+        scales = (torch.tensor(0.5, device=dev),) * 2
+    k, v = k.to(dev), v.to(dev)
+    memory = torch.empty((bs - 1) * stride + 65536, dtype=k.dtype, device=dev)
+    far = [memory.as_strided(k.shape, (4096, stride, d, 1), at) for at in (0, 32768)]
+    for view, pool in zip(far, (k, v)):
+        view.copy_(pool)
+    tables = torch.tensor([[3, 1, 5], [0, 4, 2]], dtype=torch.int32, device=dev)
+    lengths = torch.tensor([48, 37], dtype=torch.int32, device=dev)
+    plain, comp = pkg.MI355XPagedAttention(), pkg.MI355XPagedAttention(compensate=True)
+    q = torch.randn(130, hq, d, generator=g).to(torch.bfloat16).to(dev)
+
+    def windows(n):
+        return torch.tensor([0, n, 2 * n], dtype=torch.int32, device=dev)
+
+    for name, call in (
+            ("decode", lambda a, b: plain(q[:2], a, b, tables, lengths, *scales)),
+            ("window", lambda a, b: plain.prefill(q[:10], a, b, tables, lengths, windows(5), 5, *scales)),
+            ("compensated", lambda a, b: comp.prefill(q[:10], a, b, tables, lengths, windows(5), 5,
+                                                      *scales)),
+            ("prefill", lambda a, b: plain.prefill(q, a, b, tables, lengths, windows(65), 65, *scales))):
+        assert torch.equal(call(*far).view(torch.int16), call(k, v).view(torch.int16)), name
+
+
 def test_window_store_of_many_padded_windows(kernel, pkg, dev):
     """A ragged batch whose longest window could hold 2^20 rows: the padded windows take 2^24
     workgroups of the store ahead of the prefill tiling, more than one grid of 256 threads
