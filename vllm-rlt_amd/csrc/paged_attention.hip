@@ -285,11 +285,6 @@ struct Mfma<RLT_F16> {
   }
 };
 
-template <bool B>
-struct Flag {
-  static constexpr bool value = B;
-};
-
 // Two fp8 codes (the low or high half of w) -> packed 16-bit values of the MFMA type
 // (exact for e4m3; one gfx950 pair conversion).
 template <int QT, bool kHigh>

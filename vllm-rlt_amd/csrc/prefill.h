@@ -84,8 +84,9 @@ __device__ __forceinline__ int v_slot(int r, int piece) {
 // LDS writes from the buffers read meanwhile, made every transpose read wait for all loads
 // in flight, and every K read for all reads before it; the caller waits with wait_loads().
 // The s_nop covers a base register written by the vector unit just before (5 wait states)
-// and M0's own wait state.  (M0 is reserved: the compiler keeps no value in it, and sets it
-// right before each instruction of its own that reads it.)
+// and M0's own wait state.  (M0 is a reserved register, which the compiler lets no clobber list
+// name.  No other instruction of this kernel reads it; one that did -- the compiler may set it
+// once for several of its own -- would need it saved and restored here.)
 __device__ __forceinline__ uint32_t lds_offset(const void* p) {
   return (uint32_t)(uintptr_t)(lds_void*)p;
 }
