@@ -166,6 +166,10 @@ __global__ __launch_bounds__(kPfThreads, 2) void rlt_prefill_kernel(AttnParams P
   // fewer registers)
   constexpr int kAheadK = FP8 ? 2 : 4;
   constexpr int kAheadV = FP8 ? 2 : 3;
+  // fp8 V is loaded with K where the registers hold both (after K's pieces have left theirs, V's
+  // latency shows on cold keys: 8 windows of up to 130 rows behind 3000, 16 heads of 64 dims,
+  // 80.7 -> 62.3 us; with per-vector scales it took 88.6 -> 93.1)
+  constexpr bool kEarlyV = SM == 1 && D <= 64;
   constexpr int NC = FP8 ? FJ : 1;  // 16-position groups a wave loads from per tile
   __shared__ L sh;
   const int t = threadIdx.x, lane = t & 63, l32 = lane & 31, h = lane >> 5;
@@ -237,17 +241,21 @@ __global__ __launch_bounds__(kPfThreads, 2) void rlt_prefill_kernel(AttnParams P
   const int32_t* table = P.tables + (int64_t)seq * P.table_stride;
   const int dq = kPfKeys / P.block_size, dr = kPfKeys % P.block_size;
   // block id and offset of position pos: entries outside the pool read block 0
-  auto pool_block = [&](int32_t e) { return (int64_t)((e >= 0 && e < P.num_blocks) ? e : 0); };
-  auto lookup = [&](int pos, int64_t& blk, int& off) {
-    blk = pool_block(table[min(pos / P.block_size, P.table_width - 1)]);
-    off = pos % P.block_size;
+  auto pool_block = [&](int32_t e) { return (e >= 0 && e < P.num_blocks) ? e : 0; };
+  // the tile's row whose block the wave's c-th cursor follows: the first of the 16-position
+  // group of its c-th access (UB), or, in lane i, the row that access i / ROWS_PER_LD of lanes
+  // (i % ROWS_PER_LD) SLOTS .. reads (one lookup per row and wave; a lookup with its divisions
+  // per access took 44.3 us where this takes 30.0, 4 prompts of 300-500 rows at block size 8)
+  auto cursor_row = [&](int c) {
+    const int i = UB ? ROWS_PER_LD * c : lane & 15;
+    const int r = FP8 ? i / ROWS_PER_LD * (kPfThreads / SLOTS) + w * ROWS_PER_LD + i % ROWS_PER_LD
+                      : 16 * w + i;
+    return UB ? r & ~15 : r;
   };
-  // first row (within the tile) of the 16-position group of the wave's c-th access
-  auto group_row = [&](int c) { return FP8 ? (c * (kPfThreads / SLOTS) + w * (64 / SLOTS)) & ~15 : 16 * w; };
   // blocks and offsets of the K tile loaded last; the cursor holds the next tile's
-  TileCursor cur[UB ? NC : 1];
-  int64_t kblk[UB ? NC : 1] = {};
-  int koff[UB ? NC : 1] = {};
+  constexpr int CUR = UB ? NC : 1;
+  TileCursor cur[CUR];
+  int kblk[CUR] = {}, koff[CUR] = {};
   // per-vector scales: wave 0 stages the keys' (with the K tile), wave 1 the values'
   TileCursor scur;
   const bool scale_wave = SM == 2 && w < 2;
@@ -301,38 +309,29 @@ __global__ __launch_bounds__(kPfThreads, 2) void rlt_prefill_kernel(AttnParams P
     }
   };
   constexpr int NJ = FP8 ? FJ : LD;
-  // row (within the tile) that this lane's j-th access reads
-  auto lane_row = [&](int j) { return FP8 ? (j * kPfThreads + t) / SLOTS : 16 * w + ROWS_PER_LD * j + ld_row; };
   // the cursor's tile becomes the K tile to load, and the next entry is read (before any
   // load of this iteration is in flight: the entry's use would wait for all of them)
   auto next_blocks = [&]() {
-    if constexpr (UB) {
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        kblk[c] = pool_block(__builtin_amdgcn_readfirstlane(cur[c].next));
-        koff[c] = cur[c].off;
-        cur[c].advance(P, table, dq, dr);
-      }
+    for (int c = 0; c < CUR; ++c) {
+      kblk[c] = pool_block(UB ? __builtin_amdgcn_readfirstlane(cur[c].next) : cur[c].next);
+      koff[c] = cur[c].off;
+      cur[c].advance(P, table, dq, dr);
     }
   };
-  auto load_k = [&](int tile, int b) {
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      int64_t blk = kblk[UB && FP8 ? j : 0];
-      int off = koff[UB && FP8 ? j : 0];
-      if constexpr (!UB) lookup(tile * kPfKeys + lane_row(j), blk, off);
-      load_k_piece(b, j, blk, off);
-    }
+  // block and offset of this lane's j-th access among the wave's
+  auto access = [&](const int (&x)[CUR], int j) {
+    if (UB) return x[FP8 ? j : 0];
+    return __builtin_amdgcn_ds_bpermute(4 * (ROWS_PER_LD * j + lane / SLOTS), x[0]);
   };
-  // V of `tile` into buffer b, from the blocks `blk`, `off` that its K was loaded from
-  auto load_v = [&](int tile, int b, const int64_t (&blks)[UB ? NC : 1], const int (&offs)[UB ? NC : 1]) {
+  auto load_k = [&](int b) {
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      int64_t blk = blks[UB && FP8 ? j : 0];
-      int off = offs[UB && FP8 ? j : 0];
-      if constexpr (!UB) lookup(tile * kPfKeys + lane_row(j), blk, off);
-      load_v_piece(b, j, blk, off);
-    }
+    for (int j = 0; j < NJ; ++j) load_k_piece(b, j, access(kblk, j), access(koff, j));
+  };
+  // V of a tile into buffer b, from the blocks `blks`, `offs` that its K was loaded from
+  auto load_v = [&](int b, const int (&blks)[CUR], const int (&offs)[CUR]) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) load_v_piece(b, j, access(blks, j), access(offs, j));
   };
   // the scales of the cursor's tile, read into a register (wave 0 keys, wave 1 values)
   auto load_scale = [&](int tile) {
@@ -536,14 +535,12 @@ __global__ __launch_bounds__(kPfThreads, 2) void rlt_prefill_kernel(AttnParams P
 
   if (kt0 < kt1) {
     // ---- first tiles: K and V of kt0, K of kt0 + 1, the scores of kt0
-    if constexpr (UB) {
 #pragma unroll
-      for (int c = 0; c < NC; ++c) cur[c].start(P, table, kt0 * kPfKeys + group_row(c));
-    }
+    for (int c = 0; c < CUR; ++c) cur[c].start(P, table, kt0 * kPfKeys + cursor_row(c));
     if (scale_wave) scur.start(P, table, kt0 * kPfKeys + lane);
     next_blocks();
-    load_k(kt0, 0);
-    load_v(kt0, 0, kblk, koff);
+    load_k(0);
+    load_v(0, kblk, koff);
     if constexpr (FP8) {
       put_k(0);
       put_v(kt0, 0);
@@ -554,7 +551,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void rlt_prefill_kernel(AttnParams P
     }
     if (kt0 + 1 < kt1) {
       next_blocks();
-      load_k(kt0 + 1, 1);
+      load_k(1);
       if constexpr (FP8) {
         put_k(1);
         if (scale_wave && w == 0) {
@@ -580,26 +577,25 @@ __global__ __launch_bounds__(kPfThreads, 2) void rlt_prefill_kernel(AttnParams P
     // one tile: `cur_s` are its scores, b its buffers; the next tile's scores go to `next_s`
     auto step = [&](int tile, int b, f32x16 (&cur_s)[2], f32x16 (&next_s)[2]) {
       const bool more = tile + 2 < kt1;
-      int64_t vblk[UB ? NC : 1];
-      int voff[UB ? NC : 1];
+      int vblk[CUR], voff[CUR];
 #pragma unroll
-      for (int c = 0; c < (UB ? NC : 1); ++c) {
+      for (int c = 0; c < CUR; ++c) {
         vblk[c] = kblk[c];
         voff[c] = koff[c];
       }
       if (more) next_blocks();
-      if constexpr (!FP8) load_v(tile + 1, b ^ 1, vblk, voff);
-      if (more) load_k(tile + 2, b);
+      if constexpr (!FP8) load_v(b ^ 1, vblk, voff);
+      if (more) load_k(b);
+      if constexpr (kEarlyV) load_v(b ^ 1, vblk, voff);
       if (SM == 2 && (w == 1 || (w == 0 && more))) load_scale(tile + (w == 0 ? 2 : 1));
       uint32_t p[16];
       scores(next_s, b ^ 1, [&](int c) {
         quads(c, NQS, [&](int g) { weigh_quad(cur_s, p, g, b); });
       });
       if constexpr (FP8) {
-        // K's raw pieces leave their registers before V's arrive (both buffers are free
-        // for the whole iteration)
+        // (both buffers are free for the whole iteration)
         if (more) put_k(b);
-        load_v(tile + 1, b ^ 1, vblk, voff);
+        if constexpr (!kEarlyV) load_v(b ^ 1, vblk, voff);
       }
       scale_scores(next_s, b ^ 1);
       mask(next_s, tile + 1);
