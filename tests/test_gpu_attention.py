@@ -1134,16 +1134,9 @@ def test_packed_window_shape_selects_compensation(pkg, dev):
                                   packed_window_shape=shape).kernel.compensate
 
 
-@pytest.mark.parametrize("kv", ["same", "fp8", "fp8_vector"])
-@pytest.mark.parametrize("d,hkv", [(64, 1), (96, 3), (128, 2), (128, 8)])
-def test_long_window_store_ragged_rows(kernel, pkg, dev, kv, d, hkv):
-    """The window store ahead of the prefill tiling on ragged windows (none, one row, a
-    window that starts at position 0, one past a workgroup's vectors): exactly the bits of
-    store_kv / store_fp8, and no other byte of the pool touched."""
-    _say("ragged window store", kv, d, hkv)
+def _ragged_store(kernel, pkg, dev, kv, d, hkv, q_lens, lengths):
     g = torch.Generator().manual_seed(d + hkv)
-    dtype, bs, q_lens = torch.bfloat16, 16, [64, 0, 1, 33, 131, 70]
-    lengths = [64, 40, 7, 2049, 500, 513]
+    dtype, bs = torch.bfloat16, 16
     pages = sum(-(-x // bs) for x in lengths) + 4
     tables = random_tables(lengths, bs, pages, g)
     rows = sum(q_lens)
@@ -1171,7 +1164,7 @@ def test_long_window_store_ragged_rows(kernel, pkg, dev, kv, d, hkv):
                       fixed_scale=0.0375 if kv == "fp8" else None)
         args = tuple(scales) if kv == "fp8_vector" else (torch.tensor(0.0375, device=dev),) * 2
     cu = torch.tensor([0] + torch.cumsum(torch.tensor(q_lens), 0).tolist(), dtype=torch.int32)
-    assert kernel.uses_prefill_tiling(dtype, pools[0].dtype, d, max(q_lens))
+    assert kernel.uses_prefill_tiling(dtype, pools[0].dtype, d, max(q_lens)) == (max(q_lens) >= 64)
     kernel.prefill_store(q, k_new, v_new, *pools, tables.to(dev),
                          torch.tensor(lengths, dtype=torch.int32).to(dev), cu.to(dev),
                          max(q_lens), *args)
@@ -1242,6 +1235,28 @@ def test_window_store_of_many_padded_windows(kernel, pkg, dev):
     for got, ref in zip(pools, want):
         assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
     assert torch.equal(out, kernel.prefill(q, *want, *args, max(q_lens)))
+
+
+@pytest.mark.parametrize("kv", ["same", "fp8", "fp8_vector"])
+@pytest.mark.parametrize("d,hkv", [(64, 1), (96, 3), (128, 2), (128, 8)])
+def test_long_window_store_ragged_rows(kernel, pkg, dev, kv, d, hkv):
+    """The window store ahead of the prefill tiling on ragged windows (none, one row, a
+    window that starts at position 0, one past a workgroup's vectors): exactly the bits of
+    store_kv / store_fp8, and no other byte of the pool touched."""
+    _say("ragged window store", kv, d, hkv)
+    _ragged_store(kernel, pkg, dev, kv, d, hkv, [64, 0, 1, 33, 131, 70], [64, 40, 7, 2049, 500, 513])
+
+
+@pytest.mark.parametrize("kv", ["same", "fp8", "fp8_vector"])
+@pytest.mark.parametrize("d,hkv", [(64, 1), (96, 3), (128, 2), (256, 1)])
+@pytest.mark.parametrize("longest", [63, 32, 31, 4])
+def test_fused_store_ragged_rows(kernel, pkg, dev, kv, d, hkv, longest):
+    """The verify kernels' fused store on windows of every remainder of its four rows a step,
+    across chunks and from position 0, on both sides of the line from which fp8 stores keep
+    neighbouring heads apart: the same."""
+    _say("ragged fused store", kv, d, hkv, longest)
+    q_lens = [longest, 0, 1, longest - 1, 2, longest - 2, 3]
+    _ragged_store(kernel, pkg, dev, kv, d, hkv, q_lens, [longest, 40, 7, 2049, 513, 1030, 1025])
 
 
 @pytest.mark.parametrize("kv,d", [("same", 96), ("fp8_vector", 64), ("fp8_vector", 128)])

@@ -509,48 +509,61 @@ __device__ __forceinline__ bool store_rows(const AttnParams& P, int seq, int kvh
     const int64_t h_stride = is_v ? P.v_head_stride : P.k_head_stride;
     float* scales = const_cast<float*>(is_v ? P.v_scale : P.k_scale);
     const float fixed = SM == 1 ? scales[0] : 0.f;
-    for (int i = i_lo; i < i_hi; ++i) {  // wave-uniform: the lanes reduce together
-      const int pos = position(i);
-      if (pos < p0 || pos >= p1 || pos < 0) continue;
-      const int32_t e = block(pos);
-      if (e < 0 || e >= P.num_blocks) continue;
-      float x[8];
-      float amax = 0.f;
-      if (piece < kPieces) {
-        const int64_t row = (int64_t)(sv.q_begin + i) * P.new_row_stride + (int64_t)kvh * P.new_head_stride;
-        const uint4 raw = ((const uint4*)(src + row))[piece];
-        const uint32_t w4[4] = {raw.x, raw.y, raw.z, raw.w};
+    // kAtOnce rows a step, their loads in flight together (one row at a time, a window of 64
+    // rows waited out 64 rows' latencies, about 65 us of its wave: 8 windows of up to 63 rows
+    // behind 3000, 55 heads of 96 dims, 242 -> 214 us).  Wave-uniform: the lanes reduce together.
+    constexpr int kAtOnce = 4;
+    for (int i0 = i_lo; i0 < i_hi; i0 += kAtOnce) {
+      uint4 raw[kAtOnce];
+      int32_t entry[kAtOnce];
+      int64_t off[kAtOnce];
+#pragma unroll
+      for (int r = 0; r < kAtOnce; ++r) {
+        const int i = i0 + r;
+        const int pos = i < i_hi ? position(i) : -1;
+        const bool live = pos >= p0 && pos < p1 && pos >= 0;
+        entry[r] = live ? block(pos) : -1;
+        off[r] = pos % P.block_size;
+        raw[r] = make_uint4(0, 0, 0, 0);
+        if (live && piece < kPieces)
+          raw[r] = ((const uint4*)(src + (int64_t)(sv.q_begin + i) * P.new_row_stride +
+                                   (int64_t)kvh * P.new_head_stride))[piece];
+      }
+#pragma unroll
+      for (int r = 0; r < kAtOnce; ++r) {
+        if (entry[r] < 0 || entry[r] >= P.num_blocks) continue;
+        const uint32_t w4[4] = {raw[r].x, raw[r].y, raw[r].z, raw[r].w};
+        float x[8];
+        float amax = 0.f;  // (lanes past the vector hold zeros)
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          if (QT == RLT_BF16) {
-            x[2 * u] = __uint_as_float(w4[u] << 16);
-            x[2 * u + 1] = __uint_as_float(w4[u] & 0xffff0000u);
-          } else {
-            x[2 * u] = f16_bits_to_f32((uint16_t)(w4[u] & 0xffffu));
-            x[2 * u + 1] = f16_bits_to_f32((uint16_t)(w4[u] >> 16));
+          x[2 * u] = Mfma<QT>::lo_f32(w4[u]);
+          x[2 * u + 1] = Mfma<QT>::hi_f32(w4[u]);
+        }
+        float scale = fixed;
+        if (SM == 2) {
+#pragma unroll
+          for (int u = 0; u < 8; ++u) amax = rlt_fp8::nan_max(amax, fabsf(x[u]));
+          // the row's maximum over the 32 lanes of its half of the wave
+#pragma unroll
+          for (int o = 16; o >= 1; o >>= 1) amax = rlt_fp8::nan_max(amax, __shfl_xor(amax, o, RLT_WAVE));
+          scale = rlt_fp8::dynamic_scale(amax);
+        }
+        if (piece < kPieces) {
+          uint32_t lo = 0, hi = 0;
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            lo |= rlt_fp8::encode(x[u], scale) << (8 * u);
+            hi |= rlt_fp8::encode(x[4 + u], scale) << (8 * u);
           }
+          *(uint2*)(pool + (int64_t)entry[r] * b_stride + off[r] * t_stride + (int64_t)kvh * h_stride +
+                    8 * piece) = make_uint2(lo, hi);
         }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) amax = rlt_fp8::nan_max(amax, fabsf(x[u]));
+        if (SM == 2 && piece == 0)
+          scales[(int64_t)entry[r] * P.s_block_stride + off[r] * P.s_token_stride +
+                 (int64_t)kvh * P.s_head_stride] = scale;
+        stored = true;
       }
-      // the row's maximum over the 32 lanes of its half of the wave
-#pragma unroll
-      for (int o = 16; o >= 1; o >>= 1) amax = rlt_fp8::nan_max(amax, __shfl_xor(amax, o, RLT_WAVE));
-      const float scale = SM == 2 ? rlt_fp8::dynamic_scale(amax) : fixed;
-      const int64_t off = (int64_t)(pos % P.block_size);
-      if (piece < kPieces) {
-        uint32_t lo = 0, hi = 0;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          lo |= rlt_fp8::encode(x[u], scale) << (8 * u);
-          hi |= rlt_fp8::encode(x[4 + u], scale) << (8 * u);
-        }
-        *(uint2*)(pool + (int64_t)e * b_stride + off * t_stride + (int64_t)kvh * h_stride + 8 * piece) =
-            make_uint2(lo, hi);
-      }
-      if (SM == 2 && piece == 0)
-        scales[(int64_t)e * P.s_block_stride + off * P.s_token_stride + (int64_t)kvh * P.s_head_stride] = scale;
-      stored = true;
     }
   }
   return stored;
@@ -1945,7 +1958,13 @@ int attention_impl(const void* q, int64_t q_row_stride, int64_t q_head_stride,
     P.head_groups = num_kv_heads;
     const int64_t pairs = (int64_t)num_seqs * P.rowgroups;
     P.persistent = pairs <= kMaxPairs;
-    P.shared_lines = num_kv_heads > 1 &&
+    // (not with an fp8 store of 32 rows or more: quantizing them is a good part of its unit's time,
+    // and neighbouring heads of the chunk that holds the window put such units on the same
+    // workgroups.  8 windows of up to 24 / 32 / 48 / 63 rows behind 3000, 55 heads of 96, apart
+    // and together: 111 / 130 / 198 / 214 and 111 / 130 / 238 / 272 us, 24 at 2000: 207 / 220 / 394
+    // / 422 and 204 / 233 / 402 / 439; 24 windows of up to 5 / 16 rows: 162 / 188 and 147 / 178)
+    const bool long_store = store && kv_dtype == RLT_FP8_E4M3 && max_q_len >= 32;
+    P.shared_lines = num_kv_heads > 1 && !long_store &&
                      ((k_head_stride * kv_elt) % 128 != 0 || (v_head_stride * kv_elt) % 128 != 0 ||
                       (scale_mode == 2 && s_head_stride * 4 < 128));
     int64_t wgs = (int64_t)num_seqs * P.rowgroups * num_kv_heads * P.max_chunks;
