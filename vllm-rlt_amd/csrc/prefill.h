@@ -21,11 +21,12 @@
 // What bounds it: a 128-row tile needs ~1030 cycles of a SIMD's matrix core, ~600 of its
 // vector unit and ~1020 of the CU's LDS reads (32 KB a wave: every wave reads the whole K
 // and V tile), so the three overlap or add up.  bf16, D = 128, 16 / 4 heads, against the
-// unpipelined 16x16x32 form of the same split: 8 x 2048 prompts 260 -> 155 us (530 -> 890
-// TFLOP/s), 1 x 8192 400 -> 278 (687 -> 990), 6 x 470-token chunks behind a prefix 88 -> 52;
-// fp8 8 x 2048 276 -> 182 us, with per-vector scales 311 -> 213 (a large bf16 matrix product
-// reaches 1360 TFLOP/s here).  The time without overlap went into waits: the transpose
-// reads waited for the next tile's loads, the matrix cores for the softmax.
+// unpipelined 16x16x32 form of the same split (graph replays, two boxes): 8 x 2048 prompts 254
+// -> 176-179 us (541 -> 770-780 TFLOP/s), 4 x 4096 431 -> 296-306, 1 x 8192 400 -> 292-306
+// (687 -> 897-943), D = 96 8 x 2048 271 -> 143-149, fp8 8 x 2048 294 -> 203-210; 6 chunks of up to
+// 512 rows in fp8 with per-vector scales behind a prefix, store included, 162 -> 110 (a large
+// bf16 matrix product reaches 1360 TFLOP/s here).  The time without overlap went into waits:
+// the transpose reads waited for the next tile's loads, the matrix cores for the softmax.
 #pragma once
 
 constexpr int kPfWaves = 4;                // waves per workgroup (sharing each staged tile)

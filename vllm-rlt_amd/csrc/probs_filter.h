@@ -15,11 +15,12 @@
 //      after the last kept one), and forms what the acceptance sampler or the draft step
 //      wants of it.
 //
-// What bounds it: the slice launch's instructions per column and its reductions (24 us of 80
-// rows of 151936 fp32 logits, at four workgroups a CU; write 15, row 13 to 22: its chain of
-// dependent reads).  80 such rows, bf16, top-k and top-p mixed, with the acceptance: 210 ->
-// 104 us against one workgroup per row; top-p 0.9 of 160 fp32 rows 150 -> 80 us, of 5 rows 88 ->
-// 25.  The earlier forms of this split that were measured: the cut and the ranking repeated
+// What bounds it: the slice launch's instructions per column and its reductions (19 us of 80
+// rows of 151936 fp32 logits at top-p 0.9, at four workgroups a CU; write 15; row 13, its chain of
+// dependent reads).  80 bf16 rows, top-k and top-p mixed, in an acceptance call: slices and the
+// drafts' sums 26, row 36 (the chain three times over, one search per cut), write 18; the call
+// 210 -> 102 us against one workgroup per row.  Top-p 0.9 of 160 fp32 rows 150 -> 76 us, of 8 rows
+// 88 -> 27.  The earlier forms of this split that were measured: the cut and the ranking repeated
 // by every slice's workgroup (the launches were latency chains of 10 us at four workgroups a
 // CU: 1.5x slower), the row launch reading whole rows instead of the slices that hold tokens
 // of the cut bins (608 KB by one CU: 5 to 10 us slower).
