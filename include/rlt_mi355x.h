@@ -290,7 +290,7 @@ int rlt_row_mass_f32(const float* x, int64_t rows, int64_t vocab, float* out, vo
  * threshold within that rounding.
  * The plan queries give the bytes of a call with these filters (0: none needed); the queries
  * without a plan give the largest of any call's, so 256 MiB and more for many rows of more
- * than 81920 columns, where a call that filters no row needs 16 bytes per 4096 columns of one.
+ * than 81920 columns, where a call that filters no row needs 24 bytes per 4096 columns of one.
  */
 size_t rlt_probabilities_plan_workspace_size(int64_t rows, int64_t argmax_rows, int64_t vocab,
                                              int64_t max_top_k, int32_t apply_top_p);
